@@ -43,6 +43,8 @@ template <int D_>
 struct B16Traits {
     static constexpr int DP = D_;
     using elem = u16;
+    using gelem = u16;
+    static constexpr int WAVES_PER_EU = DP == 32 ? 5 : DP == 64 ? 4 : 2;
     using chunk = uint4;
     static constexpr int KSTR = DP + 8;  // rows 16*(DP/8+1) bytes apart
     // Row-major V rows: a pitch of DP + 16 (8 dwords past a multiple of 32)
@@ -64,7 +66,7 @@ struct B16Traits {
             q.v[s] = as_bf16x8(valid ? *reinterpret_cast<const uint4*>(p + 8 * s) : uint4{0u, 0u, 0u, 0u});
     }
 
-    __device__ __forceinline__ static float score_scale(float qscale) { return qscale; }
+    __device__ __forceinline__ static float score_scale(const QReg&, float qscale) { return qscale; }
     __device__ __forceinline__ static chunk from_u32x4(u32x4 v) { return uint4{v[0], v[1], v[2], v[3]}; }
 
     template <bool VEC>
@@ -116,17 +118,24 @@ struct B16Traits {
             }
         }
     }
-    __device__ __forceinline__ static void pv(const VReg& vr, const floatx16& p, floatx16* o, int, int) {
-        bf16x8 pb[2];
+    struct PReg {
+        bf16x8 s[2];
+    };
+    template <bool SCALED = false>
+    __device__ __forceinline__ static PReg to_p(const floatx16& p) {
+        PReg pb;
 #pragma unroll
         for (int s = 0; s < 2; ++s)
 #pragma unroll
-            for (int j = 0; j < 8; ++j) pb[s][j] = (__bf16)p[8 * s + j];
+            for (int j = 0; j < 8; ++j) pb.s[s][j] = (__bf16)p[8 * s + j];
+        return pb;
+    }
+    __device__ __forceinline__ static void pv(const VReg& vr, const PReg& pb, floatx16* o, int, int) {
 #pragma unroll
         for (int db = 0; db < DP / 32; ++db)
 #pragma unroll
             for (int s = 0; s < 2; ++s)
-                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(vr.v[db][s]), pb[s], o[db], 0, 0, 0);
+                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(vr.v[db][s]), pb.s[s], o[db], 0, 0, 0);
     }
 };
 

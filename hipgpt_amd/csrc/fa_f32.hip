@@ -1,9 +1,10 @@
-// fa_f32.hip -- exact fp32 attention forward on gfx950 MFMA.
+// fa_f32.hip -- fp32 attention forward on gfx950 MFMA.
 //
 // Replaces flash_attention_kernel<32|64> and multihead_attention_kernel_fallback
 // (HipGPT src/hip_kernels.cpp:263-325, :329-402) for head dims up to 128
 // (D = 16, 48, 96, ... run zero-padded to the next of 32/64/128).  The kernel
-// body is fa_kernel.h; this file supplies the fp32 operand traits:
+// body is fa_kernel.h; this file supplies the operand traits -- F32HalfTraits
+// below, and F32Traits, the fp32 MFMA ones it falls back to:
 //   * S^T = K Q^T on v_mfma_f32_32x32x2_f32.  Q is held in registers,
 //     pre-scaled by scale*log2(e) (so scores are already in the log2
 //     domain).  Lane (c, h) takes the contraction indices d = h*DP/2 + s:
@@ -19,7 +20,6 @@
 //   D[m][n]: register r holds D[8*(r/4) + 4*h + (r%4)][c]
 #include "common.h"
 #include "fa_kernel.h"
-#include "fa_resident.h"
 #include "kernels.h"
 
 namespace hipgpt {
@@ -32,6 +32,7 @@ template <int DP_, bool VPRE_ = (DP_ <= 32), int SRES_ = (DP_ == 32 ? 4 : 0)>
 struct F32Traits {
     static constexpr int DP = DP_;
     using elem = float;
+    using gelem = float;
     using chunk = floatx4;
     static constexpr int KSTR = DP + 4;
     static constexpr int VTP = BK + 4;
@@ -65,7 +66,7 @@ struct F32Traits {
     __device__ __forceinline__ static chunk from_u32x4(u32x4 v) { return __builtin_bit_cast(chunk, v); }
 
     // Q already carries scale*log2(e).
-    __device__ __forceinline__ static float score_scale(float) { return 1.0f; }
+    __device__ __forceinline__ static float score_scale(const QReg&, float) { return 1.0f; }
 
     template <bool VEC>
     __device__ __forceinline__ static chunk load_chunk(const float* base, int64_t rowoff, int cc, int D, bool ok) {
@@ -134,6 +135,9 @@ struct F32Traits {
 #pragma unroll
             for (int db = 0; db < DP / 32; ++db) load_block(vr.v[VPRE ? db : 0], Vt, db, c, hf);
     }
+    using PReg = floatx16;
+    template <bool SCALED = false>
+    __device__ __forceinline__ static const floatx16& to_p(const floatx16& p) { return p; }
     __device__ __forceinline__ static void pv(const VReg& vr, const floatx16& p, floatx16* o, int c, int hf) {
 #pragma unroll
         for (int db = 0; db < DP / 32; ++db) {
@@ -153,47 +157,204 @@ struct F32Traits {
     }
 };
 
-// Workgroup shape per padded head dim: NQS query sub-blocks x NKS key splits,
-// measured on MI355X with waves ranked by SIMD: D=32 2x2 (c1), D=64 4x2 (c3),
-// D=128 8x1 (c4) -- the larger head dims run 2 waves per SIMD, and more query
-// sub-blocks per workgroup share each K/V stage.
-template <int DP, int NQS, int NKS, bool CAUSAL_INST = true>
-hipError_t launch_dp(const AttnArgs& a, bool causal, bool probs, bool vec, hipStream_t s) {
-    return vec ? fa::launch_fa_flags<F32Traits<DP>, NQS, NKS, true, CAUSAL_INST>(a, causal, probs, s)
-               : fa::launch_fa_flags<F32Traits<DP>, NQS, NKS, false, CAUSAL_INST>(a, causal, probs, s);
+typedef short v4i16 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
+
+// The products on operands split into two fp16 terms (split.h), the traits
+// every problem runs unless its data need F32Traits (`exact`).  Tiles are two
+// row-major planes; operand layouts as in fa_bf16.hip (v_mfma_f32_32x32x16).
+//   Q: each row is scaled by the power of two that brings its largest
+//     magnitude to [2^7, 2^8), taken out of the scores by score_scale.
+//   K: times 2^6.  Whatever K's own scale, its terms are off by at most
+//     max(2^-24 |k|, 2^-31), so a score (log2 units) by a few 2^-31 |q|: the
+//     rows where that is not far below the rounding of the exponential have
+//     an entry of 16 or more (big()) and take the exact traits.
+//   V: times 2^8; exact traits if every |v| is below 2^-9.
+//   P: below 2^15 (kHalfPShift, kHalfPScale).
+// What overflows fp16 (|k| >= 1023, |v| >= 255) or is not finite ends in O as
+// inf or NaN and takes the exact traits.
+// B8 H12 S1024 D64 causal 124 -> 57 us, B4 H16 S2048 D128 causal 577 -> 219,
+// B32 H8 S256 D32 causal 15.6 -> 11.2, with probs unmasked 30.0 -> 22.9; error
+// against 64 bits 2.8e-7 -> 2.5e-7, 4.5e-7 -> 3.1e-7, 1.8e-7 -> 1.7e-7,
+// 4.2e-7 -> 3.6e-7.
+template <int DP_, int SRES_ = 0>
+struct F32HalfTraits {
+    static constexpr int DP = DP_;
+    using elem = unsigned short;
+    using gelem = float;
+    using exact = F32Traits<DP>;
+    using chunk = floatx4;
+    static constexpr int KSTR = DP + 8;
+    static constexpr int VRP = DP + 16;
+    static constexpr int KPL = BK * KSTR;  // one term's plane
+    static constexpr int VPL = BK * VRP;
+    static constexpr int KTILE = 2 * KPL;
+    static constexpr int VTILE = 2 * VPL;
+    static constexpr int WAVES_PER_EU = DP == 64 ? 3 : 2;
+    static constexpr int PROBS_RES_STAGES = SRES_;
+
+    struct QReg {
+        Half8 v[DP / 16];
+        float unscale;
+        unsigned top;  // bits of the row's largest |q|
+        __device__ __forceinline__ bool big() const { return top >= 0x41800000u; }  // 16
+    };
+
+    template <bool VEC>
+    __device__ __forceinline__ static void load_q(QReg& q, const float* qrow, int hf, bool valid, int D, float qscale) {
+        const float* p = qrow + hf * (DP / 2);
+        float x[DP / 2];
+        float mx = 0.f;
+#pragma unroll
+        for (int u = 0; u < DP / 2; u += 4) {
+            floatx4 t = {0.f, 0.f, 0.f, 0.f};
+            if (VEC) {
+                if (valid) t = *reinterpret_cast<const floatx4*>(p + u);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (valid && hf * (DP / 2) + u + i < D) t[i] = p[u + i];
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                x[u + i] = t[i] * qscale;
+                mx = fmaxf(mx, fabsf(x[u + i]));
+            }
+        }
+        mx = fa::halves_max(mx);
+        q.top = __float_as_uint(mx);
+        // the row's largest magnitude to [2^7, 2^8); rows below 2^-64 as if at 2^-64
+        const unsigned e = max(q.top >> 23, 63u);
+        const float scale = __uint_as_float((261u - e) << 23);
+        q.unscale = __uint_as_float((e - 7u) << 23) * (1.f / fa::kHalfKScale);
+#pragma unroll
+        for (int j = 0; j < DP / 16; ++j) {
+            float y[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) y[u] = x[8 * j + u] * scale;
+            q.v[j] = half8<false>(y, 1.f);
+        }
+    }
+
+    __device__ __forceinline__ static chunk from_u32x4(u32x4 v) { return __builtin_bit_cast(chunk, v); }
+    __device__ __forceinline__ static float score_scale(const QReg& q, float) { return q.unscale; }
+    template <bool VEC>
+    __device__ __forceinline__ static chunk load_chunk(const float* base, int64_t rowoff, int cc, int D, bool ok) {
+        return F32Traits<DP>::template load_chunk<VEC>(base, rowoff, cc, D, ok);
+    }
+    template <int PLANE>
+    __device__ __forceinline__ static void store_chunk(unsigned short* dst, const chunk& v, float s) {
+        uint2 w[2];
+        half_pair(v[0] * s, v[1] * s, w[0].x, w[1].x);
+        half_pair(v[2] * s, v[3] * s, w[0].y, w[1].y);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) *reinterpret_cast<uint2*>(dst + t * PLANE) = w[t];
+    }
+    __device__ __forceinline__ static void store_k_chunk(unsigned short* Kt, int r, int cc, const chunk& v) {
+        store_chunk<KPL>(Kt + r * KSTR + cc * 4, v, fa::kHalfKScale);
+    }
+    __device__ __forceinline__ static void store_vt_chunk(unsigned short* Vt, int r, int cc, const chunk& v) {
+        store_chunk<VPL>(Vt + r * VRP + cc * 4, v, fa::kHalfVScale);
+    }
+
+    __device__ __forceinline__ static floatx16 qk(const unsigned short* Kt, const QReg& q, int c, int hf) {
+        const unsigned short* kr = Kt + c * KSTR + hf * (DP / 2);
+        floatx16 s;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = 0.f;
+        Half8 k[DP / 16];
+#pragma unroll
+        for (int j = 0; j < DP / 16; ++j) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t) k[j].t[t] = *reinterpret_cast<const halfx8*>(kr + t * KPL + 8 * j);
+            s = mfma_half_small(k[j], q.v[j], s);
+        }
+#pragma unroll
+        for (int j = 0; j < DP / 16; ++j) s = mfma_f16(k[j].t[0], q.v[j].t[0], s);
+        return s;
+    }
+
+    struct VReg {
+        const unsigned short* vt;
+    };
+    __device__ __forceinline__ static void load_v(VReg& vr, const unsigned short* Vt, int, int) { vr.vt = Vt; }
+    // V terms of step s, block db: V[16s + 4hf + 0..3][db*32 + c] and the four
+    // rows eight further on, transposed by ds_read_b64_tr_b16.
+    __device__ __forceinline__ static Half8 v_terms(const unsigned short* Vt, int db, int s, int c, int hf) {
+        const int r = c & 15;
+        const unsigned short* p = Vt + (16 * s + 4 * hf + (r >> 2)) * VRP + db * 32 + (c & 16) + 4 * (r & 3);
+        Half8 v;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(p + t * VPL)));
+            const uint2 hi = __builtin_bit_cast(
+                uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(p + t * VPL + 8 * VRP)));
+            v.t[t] = __builtin_bit_cast(halfx8, uint4{lo.x, lo.y, hi.x, hi.y});
+        }
+        return v;
+    }
+    struct PReg {
+        Half8 s[2];
+    };
+    template <bool SCALED = false>
+    __device__ __forceinline__ static PReg to_p(const floatx16& p) {
+        PReg pb;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            float x[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) x[j] = p[8 * s + j];
+            pb.s[s] = half8<SCALED>(x, fa::kHalfPScale);
+        }
+        return pb;
+    }
+    __device__ __forceinline__ static void pv(const VReg& vr, const PReg& pb, floatx16* o, int c, int hf) {
+#pragma unroll
+        for (int db = 0; db < DP / 32; ++db)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) o[db] = mfma_half(v_terms(vr.vt, db, s, c, hf), pb.s[s], o[db]);
+    }
+};
+
+// Workgroup shapes, NQS query sub-blocks of 32 rows x NKS key splits, by how
+// far 128-query blocks (n128 of them over all (batch, head) pairs) fill the
+// device's 256 CUs.  Few: the keys of a row are split over up to four waves
+// and the workgroups are small, so that more CUs have work and a row's serial
+// chain is shorter.  Many: no key split (no merge, no wave idle in the
+// diagonal stages), two or three workgroups per CU.  SRES: probs rows of up
+// to SRES stages keep their scores in registers between the two sweeps.
+// us, shapes at n128 (head dim, entry, keys):
+//   D=32 causal, 256 keys: 2x2 9.2, 4x1 10.6 at 256; 14.8, 11.7 at 512; 1024
+//     keys: 1x4 13.6, 2x4 15.1, 2x2 17.8 at 64; 18.0, 15.2, 17.9 at 128; 2x2
+//     18.3, 4x1 24.7 at 256; 46.2, 41.1 at 1024.
+//   D=32 probs, 256 keys: 1x4 7.6, 2x2 9.7 at 64; 2x2 22.9, 4x1 29.1 at 512;
+//     1024 keys: 2x4 26.5, 2x2 31.2 at 128.
+//   D=64 causal, 256 keys: 1x4 10.0, 2x4 11.2, 4x2 11.7 at 64; 4x1 17.0, 4x2
+//     22.4 at 512; 1024 keys: 2x4 23.6, 2x2 27.3, 4x2 28.8 at 128; 4x2 37.7,
+//     4x1 39.9 at 384; 4x1 58.4, 4x2 68.3 at 768.
+//   D=64 probs, 256 keys: 2x2 33.9, 4x2 39.9, 4x1 45.0 at 512; 1024 keys: 2x4
+//     40.6, 4x2 49.5 at 128; 4x2 78, 4x1 90 at 256; level from 384 on.
+//   D=128 causal, 1024 keys: 2x2 51, 4x1 64, 8x1 74 at 128; 4x1 78, 8x1 81 at
+//     512; 8x1 136, 4x1 143 at 1024.  Probs, 256 keys: 2x2 22.5, 4x1 34 at
+//     128; 4x1 36, 2x2 39 at 256.
+template <int DP, int NQS, int NKS, int SRES = 0, bool VEC = true>
+hipError_t launch_shape(const AttnArgs& a, bool causal, bool probs, hipStream_t s) {
+    return fa::launch_fa_flags<F32HalfTraits<DP, SRES>, NQS, NKS, VEC>(a, causal, probs, s);
 }
 
-// D = 64 without a causal mask: where the 4 x 2 grid needs more than one
-// round of resident workgroups, 4 x 1 workgroups (the same 128 queries, no
-// key split, half the CU each, so twice as many resident).  Cache-rotated:
-// B8 H12 S1024 (768 workgroups on 512 4 x 2 slots) 206.5 -> 198.3 us, the
-// HipGPT drop-in there 324.9 -> 320.4 us.  Causal grids measured slower with
-// 4 x 1 at every size tried (c3 127 -> 140 us, B16 H12 S1024 229 -> 249,
-// c3 with probs 226 -> 245, S = 256 31.1 -> 33.0): their longest rows,
-// unsplit, set the end.
-// D = 32 causal without probs on rows of at most 256 keys (at most four
-// query blocks of 64): where the grid exceeds one round of 2 x 1 workgroups
-// (64 queries, no key split, 2 waves), those instead of 2 x 2 -- the key
-// split's merge and per-workgroup stage then cost more than its shorter
-// rows save, the dispatch balancing the many rounds.  Cache-rotated (G
-// workgroups against 2048 2 x 1 slots): c1's shape at B = 128 (G 4096)
-// 59.6 -> 54.1 us, B = 256 115.7 -> 109.0; level or slower at B = 48 / 64
-// (28.0 / 28.0, 32.5 / 32.0), with probs (B = 128: 101.9 -> 137.7), without
-// a causal mask (85.5 / 85.6), and on longer rows (S = 512 B32: 48.9 ->
-// 51.5, S = 1024 B8 47.5 -> 64.5, B32 154.8 -> 153.0); c1 itself (G 1024)
-// 16.7 -> 20.6.
-bool dp32_unsplit(const AttnArgs& a, bool causal, bool probs, bool vec) {
-    if (!causal || probs || !vec || a.Sq > 256 || a.Sk > 256) return false;
-    const int64_t grid = (int64_t)((a.Sq + 63) / 64) * a.B * a.H;
-    const int slots = fa::fa_resident_slots<F32Traits<32>, 2, 1, true, true>();
-    return slots > 0 && grid > slots;
-}
-
-bool dp64_narrow(const AttnArgs& a, bool causal) {
-    if (causal) return false;
-    const int64_t grid = (int64_t)((a.Sq + 127) / 128) * a.B * a.H;
-    const int slots = fa::fa_resident_slots<F32Traits<64>, 4, 2, false, true>();
-    return slots > 0 && grid > slots;
+// Head dims below the padded one and unaligned rows (guarded loads): two
+// shapes each, for grids that do and do not fill the device.
+hipError_t launch_guarded(const AttnArgs& a, bool causal, bool probs, int64_t n128, hipStream_t s) {
+    switch (fa_f32_padded_dim(a.D)) {
+        case 32: return launch_shape<32, 2, 2, 4, false>(a, causal, probs, s);
+        case 64:
+            return n128 <= 128 ? launch_shape<64, 2, 4, 0, false>(a, causal, probs, s)
+                               : launch_shape<64, 4, 2, 0, false>(a, causal, probs, s);
+        case 128:
+            return n128 <= 128 ? launch_shape<128, 2, 2, 0, false>(a, causal, probs, s)
+                               : launch_shape<128, 8, 1, 0, false>(a, causal, probs, s);
+        default: return hipErrorInvalidValue;
+    }
 }
 
 }  // namespace
@@ -207,74 +368,28 @@ int fa_f32_padded_dim(int D) {
     return 0;
 }
 
-// Probs rows of 193 to 256 keys at DP = 64 (all K/V tiles of a (b, h) fit one
-// workgroup's LDS) run the resident kernel: 8 waves = 256 queries per
-// workgroup, the scores kept between the sweeps.  Cache-rotated, B*H = 256:
-// S = 256 with probs 40.6 (causal) / 55.3 us (drop-in) against 50.7 / 65.0
-// for the streaming kernel.  Everything else streams: without probs the
-// streaming kernel measured 31.2 against 32.7 us at S = 256 (causal; 44.3
-// against 45.4 non-causal), 23.4 against 33.4 at S = 128 and 40.8 against
-// 55.8 at S = 192; with probs at S = 128 / 192, 35.6 / 55.6 against 41.9 /
-// 68.5 us causal and level / 73.1 against 75.4 non-causal.  At DP = 32 the
-// streaming kernel measured faster at every S (17.2 against 17.5 us at c1).
-constexpr int kResidentMinSq = 193, kResidentMaxSq = 256;
-
-// Small D <= 32 problems (at most 128 query tiles of 32 rows in all, 128 to
-// 256 keys -- HipGPT's generation call, B = 1, H = 8, S = 256, is 64 tiles):
-// the 2 x 2 workgroups would put one or two waves on a few dozen SIMDs, so
-// each query sub-block is split over 4 waves instead (1 x 4, at most two
-// stages of key tiles each, scores kept in registers with probs).  The
-// generation call 12.6 -> 9.2 us, B = 1 causal 9.5 -> 7.5 us; from 256 query
-// tiles on the two shapes measure the same, and below 128 keys a split would
-// hold no tile.  (1 x 8 measured 9.4 us on the generation call, 1 x 2 12.3,
-// 2 x 4 12.5.)
-constexpr int kSmallNqs = 1, kSmallNks = 4, kSmallMaxQtiles = 128;
-// The same split at D = 64 replaces the resident kernel (one 8-wave
-// workgroup per (b, h), latency-bound when B*H is far below the CU count)
-// up to 512 query tiles: the generation call at E = 512 (B = 1, H = 8,
-// S = 256, drop-in) 47.1 -> 12.8 us, B = 8 drop-in 52.0 -> 26.9 us, B = 8
-// causal 29.8 -> 20.3 us; at B = 16 (1024 tiles) the causal resident kernel
-// is faster (31.0 against 38.7 us).
-constexpr int kSmall64MaxQtiles = 512;
-
-hipError_t launch_fa_f32(const AttnArgs& a, bool causal, bool vec, hipStream_t stream) {
+hipError_t launch_fa_f32(const AttnArgs& a, bool causal, bool vec, hipStream_t s) {
     const bool probs = a.probs != nullptr;
-    {
-        constexpr int NQ = kSmallNqs, NK = kSmallNks, ST = 8 / NK;
-        using TS = F32Traits<32, true, ST>;
-        const int64_t qtiles = (int64_t)a.B * a.H * ((a.Sq + 31) / 32);
-        const bool small = vec && a.Sk >= 128 && a.Sk <= 256 && qtiles <= kSmallMaxQtiles;
-        if (small && fa_f32_padded_dim(a.D) == 32) {
-            if (probs)
-                return causal ? fa::launch_fa<TS, NQ, NK, true, true, true, ST>(a, stream)
-                              : fa::launch_fa<TS, NQ, NK, false, true, true, ST>(a, stream);
-            return causal ? fa::launch_fa<TS, NQ, NK, true, false, true>(a, stream)
-                          : fa::launch_fa<TS, NQ, NK, false, false, true>(a, stream);
-        }
-        using T6 = F32Traits<64, true, ST>;
-        if (vec && a.Sk >= 128 && a.Sk <= 256 && qtiles <= kSmall64MaxQtiles && fa_f32_padded_dim(a.D) == 64) {
-            if (probs)
-                return causal ? fa::launch_fa<T6, NQ, NK, true, true, true, ST>(a, stream)
-                              : fa::launch_fa<T6, NQ, NK, false, true, true, ST>(a, stream);
-            return causal ? fa::launch_fa<T6, NQ, NK, true, false, true>(a, stream)
-                          : fa::launch_fa<T6, NQ, NK, false, false, true>(a, stream);
-        }
-    }
-    // one workgroup per (b, h) and CU: only with probs and when the (b, h)
-    // pairs fill the device (at B*H = 128, S = 256 the streaming kernel
-    // measured 38.8 against 53.7 us for the drop-in); the resident kernel
-    // writes no lse
-    if (vec && probs && a.Sq >= kResidentMinSq && a.Sq <= kResidentMaxSq && !a.lse && a.D == 64 &&
-        (int64_t)a.B * a.H >= device_cus() && fa::resident_lds_bytes<F32Traits<64, true>, 8>(a) != 0)
-        return fa::launch_resident<F32Traits<64, true>, 8, 4>(a, causal, stream);
+    const int64_t n128 = (int64_t)a.B * a.H * ((a.Sq + 127) / 128);
+    const int Sk = a.Sk;
+    if (!vec) return launch_guarded(a, causal, probs, n128, s);
     switch (fa_f32_padded_dim(a.D)) {
         case 32:
-            if (dp32_unsplit(a, causal, probs, vec)) return fa::launch_fa<F32Traits<32>, 2, 1, true, false, true>(a, stream);
-            return launch_dp<32, 2, 2>(a, causal, probs, vec, stream);
+            if (n128 <= 64 && Sk > 128) return launch_shape<32, 1, 4, 2>(a, causal, probs, s);
+            if (n128 <= 128 && Sk > 256) return launch_shape<32, 2, 4, 2>(a, causal, probs, s);
+            if (n128 < 512 || probs) return launch_shape<32, 2, 2, 4>(a, causal, probs, s);
+            return launch_shape<32, 4, 1>(a, causal, probs, s);
         case 64:
-            return dp64_narrow(a, causal) ? launch_dp<64, 4, 1, false>(a, causal, probs, vec, stream)
-                                          : launch_dp<64, 4, 2>(a, causal, probs, vec, stream);
-        case 128: return launch_dp<128, 8, 1>(a, causal, probs, vec, stream);
+            if (n128 <= 64 && Sk <= 256 && Sk > 128) return launch_shape<64, 1, 4, 2>(a, causal, probs, s);
+            if (n128 <= 128) return launch_shape<64, 2, 4>(a, causal, probs, s);
+            if (probs && Sk <= 256) return launch_shape<64, 2, 2, 4>(a, causal, probs, s);
+            if (n128 <= 256 || (causal && n128 <= 512 && Sk > 512))
+                return launch_shape<64, 4, 2>(a, causal, probs, s);
+            return launch_shape<64, 4, 1>(a, causal, probs, s);
+        case 128:
+            if (n128 <= 128) return launch_shape<128, 2, 2>(a, causal, probs, s);
+            if (n128 <= 512 || probs) return launch_shape<128, 4, 1>(a, causal, probs, s);
+            return launch_shape<128, 8, 1>(a, causal, probs, s);
         default: return hipErrorInvalidValue;
     }
 }

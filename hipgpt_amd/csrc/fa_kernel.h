@@ -26,6 +26,7 @@
 
 #include "common.h"
 #include "fa_common.h"
+#include "split.h"
 
 namespace hipgpt {
 namespace fa {
@@ -60,6 +61,22 @@ constexpr int kTransOwnMinDP = 128;
 // Start stagger only for grids of at most this many query blocks per (b, h).
 constexpr int kStaggerMaxBlocks = 4;
 
+// Traits of split operands (split.h; HALF) name the fp32 MFMA traits they
+// stand in for as `exact`; a workgroup whose data are outside the range the
+// split is good for runs again with those.
+template <class TR, class = void>
+struct exact_traits { using type = void; };
+template <class TR>
+struct exact_traits<TR, std::void_t<typename TR::exact>> { using type = typename TR::exact; };
+
+// Powers of two the operands carry so that both fp16 terms keep their bits
+// (split.h); Q rows carry one of their own (F32HalfTraits::load_q).
+constexpr float kHalfPShift = 7.f;     // exponentials up to 2^(kLazyMax + 7) = 2^15 < 65504
+constexpr float kHalfPScale = 16384.f; // normalised probs (<= 1) before the split
+constexpr float kHalfKScale = 64.f;    // K: |k| < 1023
+constexpr float kHalfVScale = 256.f;   // V: |v| < 255
+constexpr float kHalfVMin = 1.f / 512; // and at least one |v| this large
+
 // SRT > 0 (probs only): when a wave's key tiles span at most SRT stages, the
 // max/sum sweep keeps every score tile in registers and the probs sweep reads
 // them back instead of recomputing Q K^T (it stages V only).
@@ -81,7 +98,10 @@ struct FaKernel {
     static constexpr int NT = NW * 64;
     static constexpr int NDB = DP / 32;
     static constexpr bool SPILL = SRT < 0;
-    using E = typename TR::elem;
+    using E = typename TR::elem;    // staged operands (LDS)
+    using GE = typename TR::gelem;  // K / V / Q in global memory
+    static constexpr bool F32IN = sizeof(GE) == 4;
+    static constexpr bool HALF = !std::is_void_v<typename exact_traits<TR>::type>;
 
     // LDS: two stage buffers of NKS (K tile + V^T tile); the end-of-kernel
     // merge reuses the same memory.
@@ -96,8 +116,9 @@ struct FaKernel {
     // the spilled scores and the probs alike (B4 H16 S2048 D128 with probs
     // 880 -> 867 us).  Unmasked there, the transpose measured slower (the
     // drop-in 1391 -> 1465 us).
-    static constexpr bool TRANS_RES = SRT > 0 && sizeof(E) == 4 && TR::KTILE >= QW * 36 && NW <= 2 * NKS;
-    static constexpr bool TRANS_OWN = PROBS && CAUSAL && SRT <= 0 && sizeof(E) == 4 && DP >= kTransOwnMinDP;
+    static constexpr bool TRANS_RES =
+        SRT > 0 && F32IN && TR::KTILE * (int)sizeof(E) >= QW * 36 * 4 && NW <= 2 * NKS;
+    static constexpr bool TRANS_OWN = PROBS && CAUSAL && SRT <= 0 && F32IN && DP >= kTransOwnMinDP;
     static constexpr int LDS_BYTES = BASE_BYTES + (TRANS_OWN ? NW * QW * 36 * 4 : 0);
     // Without probs, the first stage stages K alone: the first Q K^T waits for
     // the K rows only, V of that stage is requested once K has landed and is
@@ -105,7 +126,7 @@ struct FaKernel {
     // Cache-rotated: c1 (fp32, D = 32) 16.86 -> 16.62 us, c3-bf16 31.14 ->
     // 30.38 us; fp32 D = 64 (c3) 128.3 -> 128.8 us and D = 128 (c4) level, so
     // those keep the joint first stage.
-    static constexpr bool K_FIRST = !PROBS && (sizeof(E) == 2 || DP == 32);
+    static constexpr bool K_FIRST = !PROBS && (!F32IN || DP == 32);
     // Online-softmax sweeps with 16-byte loads test the running max through
     // the exponentials' sum (kLazySum) after each wave's first tile.
     // Cache-rotated, two interleaved repetitions: c1 16.63 -> 16.56 us, c3
@@ -114,7 +135,13 @@ struct FaKernel {
     // the c1 and c3 shapes level; results unchanged bit for bit.  The
     // guarded-load instances (padded head dims) spill registers with it
     // (25 at D = 128) and keep the max test.
-    static constexpr bool SUM_CHECK = VEC;
+    static constexpr bool SUM_CHECK = VEC && !(HALF && DP >= 128);
+    // Exponentials carry a factor 2^PSH without probs (it rides in m_run);
+    // with probs to_p<true> applies kHalfPScale.  Both, and V's, leave O in
+    // the epilogue.
+    static constexpr float PSH = HALF && !PROBS ? kHalfPShift : 0.f;
+    static constexpr float LAZY_SUM = HALF && !PROBS ? kLazySum * (float)(1 << (int)kHalfPShift) : kLazySum;
+    static constexpr float O_UNSCALE = !HALF ? 1.f : 1.f / kHalfVScale / (PROBS ? kHalfPScale : 1.f);
     // Causal grids larger than the device holds at once start their last
     // launch ranks (the shortest query blocks) as slots free, well into the
     // call, on Q rows nobody has read: each workgroup of rank r reads the Q
@@ -125,7 +152,7 @@ struct FaKernel {
     // 50.0 -> 47.2, c3 127.0 -> 126.5, fp32 B16 H12 S1024 228.6 -> 226.4;
     // fp32 D = 32 (B32 H8 S1024 155.8 -> 157.0) and D = 128 (c4 577 -> 579)
     // measured level or slower and go without.
-    static constexpr bool PF_LATE = CAUSAL && !PROBS && (sizeof(E) == 2 || DP == 64);
+    static constexpr bool PF_LATE = CAUSAL && !PROBS && (!F32IN || DP == 64);
     // Score-resident sweeps over at most two stages at D = 32 (the small
     // problems' 1 x 4 workgroups: HipGPT's generation call): K and V of both
     // stages are requested at once into the two stage buffers, so neither
@@ -142,7 +169,7 @@ struct FaKernel {
     static constexpr bool O_TRANS_PAST = MERGE_BYTES + O_SCR <= BASE_BYTES;
 
     // Global -> register staging of one stage (K and V), 16-byte chunks.
-    static constexpr int EPC = 16 / (int)sizeof(E);      // elements per chunk
+    static constexpr int EPC = 16 / (int)sizeof(GE);     // elements per chunk
     static constexpr int CPR = DP / EPC;                  // chunks per row
     static constexpr int CPS = NKS * BK * CPR;            // chunks per stage (K or V)
     static constexpr int PER = (CPS + NT - 1) / NT;
@@ -154,14 +181,15 @@ struct FaKernel {
     // guarded loads.)
     struct Stager {
         typename TR::chunk kr[PER], vr[PER];  // one stage of K and V chunks
+        mutable float vtop = 0.f;            // HALF: largest |v| stored
         int koff[PER], voff[PER];  // byte offsets of this thread's chunks from the stage's first row
         __amdgpu_buffer_rsrc_t krs, vrs;
         int kstage, vstage;        // bytes per stage of NKS*BK rows
-        const E *Kp, *Vp;
+        const GE *Kp, *Vp;
         int64_t kts, vts;
         int Sk, D;
 
-        __device__ __forceinline__ void init(const E* Kp_, const E* Vp_, int64_t kts_, int64_t vts_, int Sk_, int D_,
+        __device__ __forceinline__ void init(const GE* Kp_, const GE* Vp_, int64_t kts_, int64_t vts_, int Sk_, int D_,
                                              int tid) {
             Kp = Kp_;
             Vp = Vp_;
@@ -170,10 +198,10 @@ struct FaKernel {
             Sk = Sk_;
             D = D_;
             if (VEC) {
-                constexpr int ES = (int)sizeof(E);
-                krs = __builtin_amdgcn_make_buffer_rsrc(const_cast<E*>(Kp), 0,
+                constexpr int ES = (int)sizeof(GE);
+                krs = __builtin_amdgcn_make_buffer_rsrc(const_cast<GE*>(Kp), 0,
                                                         (int)(((int64_t)(Sk - 1) * kts + D) * ES), kBufferFlags);
-                vrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<E*>(Vp), 0,
+                vrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<GE*>(Vp), 0,
                                                         (int)(((int64_t)(Sk - 1) * vts + D) * ES), kBufferFlags);
                 kstage = (int)(NKS * BK * kts * ES);
                 vstage = (int)(NKS * BK * vts * ES);
@@ -223,12 +251,19 @@ struct FaKernel {
                 E* Kt = stage + kt * TR::KTILE;
                 E* Vt = stage + NKS * TR::KTILE + kt * TR::VTILE;
                 if (WK) TR::store_k_chunk(Kt, r, cc, kr[i]);
-                if (WV) TR::store_vt_chunk(Vt, r, cc, vr[i]);
+                if (WV) {
+                    TR::store_vt_chunk(Vt, r, cc, vr[i]);
+                    if constexpr (HALF)
+                        vtop = fmaxf(fmaxf(vtop, fmaxf(fabsf(vr[i][0]), fabsf(vr[i][1]))),
+                                      fmaxf(fabsf(vr[i][2]), fabsf(vr[i][3])));
+                }
             }
         }
     };
 
-    __device__ __forceinline__ static void run(const AttnArgs& a, unsigned char* lds_raw, int* simd_slots) {
+    // True (HALF only): this wave's results need the exact traits.
+    __device__ __forceinline__ static bool run(const AttnArgs& a, unsigned char* lds_raw, int* simd_slots,
+                                               int* v_seen = nullptr) {
         E* const lds = reinterpret_cast<E*>(lds_raw);
         const int tid = threadIdx.x;
         const int lane = tid & 63;
@@ -272,9 +307,9 @@ struct FaKernel {
         const int qi = qw0 + c;
         const int Sq = a.Sq, Sk = a.Sk, off = a.causal_off;
 
-        const E* Qp = static_cast<const E*>(a.q) + b * a.q_bs + h * a.q_hs;
-        const E* Kp = static_cast<const E*>(a.k) + b * a.k_bs + h * a.k_hs;
-        const E* Vp = static_cast<const E*>(a.v) + b * a.v_bs + h * a.v_hs;
+        const GE* Qp = static_cast<const GE*>(a.q) + b * a.q_bs + h * a.q_hs;
+        const GE* Kp = static_cast<const GE*>(a.k) + b * a.k_bs + h * a.k_hs;
+        const GE* Vp = static_cast<const GE*>(a.v) + b * a.v_bs + h * a.v_hs;
 
         // Short causal problems (a few query blocks per (batch, head), the
         // grid filling the device's resident slots) start with every workgroup loading its
@@ -303,9 +338,9 @@ struct FaKernel {
         const uint32_t* pf_ptr = nullptr;  // PF_LATE: this thread's 4 bytes of a later block's Q rows
         if (PF_LATE && a.pf_ranks > 0 && rank + a.pf_ranks < a.n_qblk) {
             const int pqb = qb_of(rank + a.pf_ranks);
-            constexpr int LPR = (DP * (int)sizeof(E) + 63) / 64;  // 64-byte pieces per row
+            constexpr int LPR = (DP * (int)sizeof(GE) + 63) / 64;  // 64-byte pieces per row
             const int row = pqb * NQS * QW + tid / LPR, piece = tid % LPR;
-            const int col = piece * (64 / (int)sizeof(E));  // inside the row's D elements only
+            const int col = piece * (64 / (int)sizeof(GE));  // inside the row's D elements only
             if (tid < NQS * QW * LPR && row < Sq && col < a.D)
                 pf_ptr = reinterpret_cast<const uint32_t*>(Qp + (int64_t)row * a.q_ts + col);
         }
@@ -320,7 +355,7 @@ struct FaKernel {
 
         typename TR::QReg qreg;
         TR::template load_q<VEC>(qreg, Qp + (int64_t)qi * a.q_ts, hf, qi < Sq, a.D, a.qscale);
-        const float sc = TR::score_scale(a.qscale);
+        const float sc = TR::score_scale(qreg, a.qscale);
 
         floatx16 o[NDB];
 #pragma unroll
@@ -331,9 +366,17 @@ struct FaKernel {
         float m_run = kMaxInit;
         float l_run = 0.f;
 
+        // the mask as a branch: selected in, it costs every tile two VALU
+        // instructions per score
+        auto mask_edge = [&](floatx16& s, int t) {
+            if (tr.edge(t, Sk, CAUSAL, qw0, off)) {
+                if constexpr (HALF) asm volatile("");
+                mask_tile<CAUSAL>(s, t * BK, hf, qi, Sk, off);
+            }
+        };
         auto tile_scores = [&](const E* stage, int t) -> floatx16 {
             floatx16 s = TR::qk(stage + (t % NKS) * TR::KTILE, qreg, c, hf);
-            if (tr.edge(t, Sk, CAUSAL, qw0, off)) mask_tile<CAUSAL>(s, t * BK, hf, qi, Sk, off);
+            mask_edge(s, t);
             return s;
         };
         auto vt_of = [&](const E* stage, int t) -> const E* {
@@ -397,6 +440,31 @@ struct FaKernel {
         };
         float* const Xown = reinterpret_cast<float*>(lds_raw + BASE_BYTES) + wave * QW * 36;
 
+        // Exponentials of a score tile with the lazy rescale: the running max is
+        // raised only when a row's tile max exceeds it by more than kLazyMax.
+        // m_run is the max less PSH, so that exponentials are at most
+        // 2^(kLazyMax + PSH).
+        auto lazy_exp = [&](floatx16& sv) -> float {
+            const float tmax = tile_max(sv) * sc;
+            if (__any(tmax > m_run + (kLazyMax + PSH))) {
+                const float m_new = vmax(m_run, tmax - PSH);
+                const float alpha = fast_exp2(m_run - m_new);
+                l_run *= alpha;
+#pragma unroll
+                for (int db = 0; db < NDB; ++db)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
+                m_run = m_new;
+            }
+            float lsum = kSumInit;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                sv[r] = fast_exp2(fmaf(sv[r], sc, -m_run));
+                lsum += sv[r];
+            }
+            return lsum;
+        };
+
         // ------------------------------------------------------------------
         // One stage of compute on LDS buffer (i & 1).  MODE 0: online softmax
         // + PV.  MODE 1: max/sum only (SPILL: and the scores stored).  MODE 2:
@@ -417,28 +485,6 @@ struct FaKernel {
             typename TR::VReg vreg;
             if (MODE != 1) TR::load_v(vreg, vt_of(cur, t), c, hf);  // in flight during the softmax
             if constexpr (MODE == 0) {
-                // lazy rescale: raise the running max only when a row's tile
-                // max exceeds it by more than kLazyMax
-                auto lazy_exp = [&](floatx16& sv) -> float {
-                    const float tmax = tile_max(sv) * sc;
-                    if (__any(tmax > m_run + kLazyMax)) {
-                        const float m_new = vmax(m_run, tmax);
-                        const float alpha = fast_exp2(m_run - m_new);
-                        l_run *= alpha;
-#pragma unroll
-                        for (int db = 0; db < NDB; ++db)
-#pragma unroll
-                            for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
-                        m_run = m_new;
-                    }
-                    float lsum = kSumInit;
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        sv[r] = fast_exp2(fmaf(sv[r], sc, -m_run));
-                        lsum += sv[r];
-                    }
-                    return lsum;
-                };
                 float ls;
                 if (!SUM_CHECK || i == 0) {  // stage 0 holds every wave's first tile
                     ls = lazy_exp(s);
@@ -451,14 +497,14 @@ struct FaKernel {
                         s[r] = fast_exp2(fmaf(s[r], sc, -m_run));
                         ls += s[r];
                     }
-                    if (__any(ls > kLazySum)) {
+                    if (__any(ls > LAZY_SUM)) {
                         asm volatile("" ::: "memory");  // re-read K: no copy of the first product stays live
                         s = tile_scores(cur, t);
                         ls = lazy_exp(s);
                     }
                 }
                 l_run += ls;  // this lane half's partial; the halves are summed after the sweep
-                TR::pv(vreg, s, o, c, hf);
+                TR::pv(vreg, TR::to_p(s), o, c, hf);
             } else if constexpr (MODE == 1) {
                 if constexpr (SPILL && TRANS_OWN)
                     store_t(Xown, prow - (int64_t)c * Sk, s, t * BK, pvec);
@@ -477,7 +523,7 @@ struct FaKernel {
                     store_t(Xown, prow - (int64_t)c * Sk, s, t * BK, pvec);
                 else if (qi < Sq)
                     store_probs_tile(prow, s, t * BK, hf, Sk, pvec);
-                TR::pv(vreg, s, o, c, hf);
+                TR::pv(vreg, TR::template to_p<true>(s), o, c, hf);
             }
         };
 
@@ -490,23 +536,7 @@ struct FaKernel {
             for (int r = 0; r < 16; ++r) s[r] = 0.f;
             if (ks >= wtiles) return s;
             s = tile_scores(lds, ks);
-            const float tmax = tile_max(s) * sc;
-            if (__any(tmax > m_run + kLazyMax)) {
-                const float m_new = vmax(m_run, tmax);
-                const float alpha = fast_exp2(m_run - m_new);
-                l_run *= alpha;
-#pragma unroll
-                for (int db = 0; db < NDB; ++db)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
-                m_run = m_new;
-            }
-            float ls = kSumInit;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                s[r] = fast_exp2(fmaf(s[r], sc, -m_run));
-                ls += s[r];
-            }
+            const float ls = lazy_exp(s);
             l_run += ls;
             return s;
         };
@@ -514,7 +544,7 @@ struct FaKernel {
             if (ks >= wtiles) return;
             typename TR::VReg vreg;
             TR::load_v(vreg, vt_of(lds, ks), c, hf);
-            TR::pv(vreg, p, o, c, hf);
+            TR::pv(vreg, TR::to_p(p), o, c, hf);
         };
 
         // Stage pipeline: stage i+1 is loaded into registers while stage i is
@@ -615,7 +645,7 @@ struct FaKernel {
                 } else {
                     if (qi < Sq) store_probs_tile(prow, p, t * BK, hf, Sk, pvec);
                 }
-                TR::pv(vreg, p, o, c, hf);
+                TR::pv(vreg, TR::template to_p<true>(p), o, c, hf);
             }
         };
         auto sweep_res = [&](auto second_tag, float mlog, float* prow, bool pvec) {
@@ -777,14 +807,28 @@ struct FaKernel {
 
         // ---------------- epilogue: O = O^T / l (wave ks == 0) ----------------
         // Row log-sum-exp (natural log) when asked for (no-probs path only):
-        // scores are in log2 units of scale * q.k, l = sum 2^(s - m).
+        // scores are in log2 units of scale * q.k, l = sum 2^(s - m) (without
+        // the factor 2^PSH, whose logarithm would cost the sum its last bits).
         if (!PROBS && a.lse && ks == 0 && hf == 0 && qi < Sq)
-            a.lse[(int64_t)bh * Sq + qi] = (m_run + log2f(l_run)) * kLn2;
+            a.lse[(int64_t)bh * Sq + qi] = ((m_run + PSH) + log2f(l_run * (1.f / (LAZY_SUM / kLazySum)))) * kLn2;
+        bool redo = false;
+        if constexpr (HALF) {
+            redo = qreg.big();
+            if (ks == 0 && qi < Sq) {
+                const float linv = O_UNSCALE * __builtin_amdgcn_rcpf(fmaxf(l_run, 1e-20f));
+                unsigned top = 0;
+#pragma unroll
+                for (int db = 0; db < NDB; ++db)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) top = max(top, __float_as_uint(o[db][r] * linv) & 0x7fffffffu);
+                redo |= top >= 0x7f800000u;  // inf or NaN
+            }
+        }
         if constexpr (O_TRANS) {
             if constexpr (!O_TRANS_PAST) __syncthreads();  // the merge's reads of the area are done
             if (ks == 0) {
                 float* const X = reinterpret_cast<float*>(lds_raw + (O_TRANS_PAST ? MERGE_BYTES : 0)) + qs * QW * 36;
-                const float linv = __builtin_amdgcn_rcpf(fmaxf(l_run, 1e-20f));
+                const float linv = O_UNSCALE * __builtin_amdgcn_rcpf(fmaxf(l_run, 1e-20f));
                 const int rr = lane >> 3, cc = 4 * (lane & 7);
                 float* const o0 = a.o + b * a.o_bs + h * a.o_hs + (int64_t)qw0 * a.o_ts;
 #pragma unroll
@@ -808,7 +852,7 @@ struct FaKernel {
                 }
             }
         } else if (ks == 0 && qi < Sq) {
-            const float linv = __builtin_amdgcn_rcpf(fmaxf(l_run, 1e-20f));
+            const float linv = O_UNSCALE * __builtin_amdgcn_rcpf(fmaxf(l_run, 1e-20f));
             float* orow = a.o + b * a.o_bs + h * a.o_hs + (int64_t)qi * a.o_ts;
 #pragma unroll
             for (int db = 0; db < NDB; ++db) {
@@ -827,6 +871,10 @@ struct FaKernel {
                 }
             }
         }
+        if constexpr (HALF) {
+            if (st.vtop >= kHalfVMin) *v_seen = 1;
+        }
+        return redo;
     }
 };
 
@@ -839,13 +887,34 @@ struct waves_per_eu { static constexpr int value = 1; };
 template <class TR>
 struct waves_per_eu<TR, std::void_t<decltype(TR::WAVES_PER_EU)>> { static constexpr int value = TR::WAVES_PER_EU; };
 
+template <class TR, int NQS, int NKS, bool CAUSAL, bool PROBS, bool VEC, int SRT>
+constexpr int min_waves_per_eu() {
+    // no more than the LDS lets a SIMD hold
+    constexpr int lds = FaKernel<TR, NQS, NKS, CAUSAL, PROBS, VEC, SRT>::LDS_BYTES + 1024;
+    constexpr int fit = 160 * 1024 / lds * NQS * NKS / 4;
+    constexpr int want = VEC ? waves_per_eu<TR>::value : 1;
+    return want < fit ? want : fit > 1 ? fit : 1;
+}
+
 template <class TR, int NQS, int NKS, bool CAUSAL, bool PROBS, bool VEC, int SRT = 0>
-__global__ __launch_bounds__(NQS* NKS * 64) __attribute__((amdgpu_waves_per_eu(VEC ? waves_per_eu<TR>::value : 1)))
+__global__ __launch_bounds__(NQS* NKS * 64)
+__attribute__((amdgpu_waves_per_eu(min_waves_per_eu<TR, NQS, NKS, CAUSAL, PROBS, VEC, SRT>())))
 void fa_fwd_kernel(AttnArgs a) {
     using K = FaKernel<TR, NQS, NKS, CAUSAL, PROBS, VEC, SRT>;
-    __shared__ __attribute__((aligned(16))) unsigned char lds[K::LDS_BYTES];
     __shared__ int simd_slots[NQS * NKS];
-    K::run(a, lds, simd_slots);
+    if constexpr (K::HALF) {
+        using KX = FaKernel<typename TR::exact, NQS, NKS, CAUSAL, PROBS, VEC, SRT>;
+        __shared__ __attribute__((aligned(16)))
+        unsigned char lds[K::LDS_BYTES > KX::LDS_BYTES ? K::LDS_BYTES : KX::LDS_BYTES];
+        __shared__ int redo, v_seen;
+        if (threadIdx.x == 0) redo = v_seen = 0;  // run's barriers order this before the stores below
+        if (K::run(a, lds, simd_slots, &v_seen)) redo = 1;
+        __syncthreads();
+        if (redo || !v_seen) KX::run(a, lds, simd_slots);
+    } else {
+        __shared__ __attribute__((aligned(16))) unsigned char lds[K::LDS_BYTES];
+        K::run(a, lds, simd_slots);
+    }
 }
 
 template <class TR, int NQS, int NKS, bool CAUSAL, bool PROBS, bool VEC, int SRT = 0>
@@ -912,7 +981,7 @@ struct probs_res_stages<TR, std::void_t<decltype(TR::PROBS_RES_STAGES)>> {
 template <class TR, int NQS, int NKS, bool VEC, bool CAUSAL_INST = true>
 hipError_t launch_fa_flags(const AttnArgs& a, bool causal, bool probs, hipStream_t s) {
     constexpr int SRT = probs_res_stages<TR>::value;
-    constexpr bool kSpill = VEC && sizeof(typename TR::elem) == 4 && TR::DP >= kScoreSpillMinDP;
+    constexpr bool kSpill = VEC && sizeof(typename TR::gelem) == 4 && TR::DP >= kScoreSpillMinDP;
     if constexpr (!CAUSAL_INST) {
         if (causal) return hipErrorInvalidValue;
     }
