@@ -101,6 +101,7 @@ struct GemmArgs {
     int seg_w;
     int64_t seg_stride;
     int out_bf16;
+    int by_xcd;  // set by the launcher: tiles numbered by XCD (xcd_remap)
 };
 // True when the 16-byte vector path applies (alignment, multiples of 4).
 bool gemm_vec_ok(const GemmArgs& g);
