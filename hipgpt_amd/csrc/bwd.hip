@@ -7,8 +7,9 @@
 //   Dq_i = sum_j P_ij (dO_i . V_j)       (= dO_i . (P V)_i)
 //   dS   = P o (dO V^T - Dq)
 //   dQ = c dS K,   dK = c dS^T Q,   dV = P^T dO
-// Head dims 32 and 64 with 16-byte aligned rows run the LDS-tiled kernels of
-// bwd_tiled.h; the kernels below serve every other problem.  Two kernels,
+// Head dims up to 128 with 16-byte aligned rows run bwd_half.h (or, at S <=
+// 256, one workgroup per (b, h): bwd_bh.h, bwd_bh64.h), 256 bwd_wide.h; the
+// kernels below serve every other problem.  Two kernels,
 // every gradient element written exactly once (no atomics, no memset):
 //   * query-stationary (one wave per 32 queries): pass 1 forms (P V)_i on
 //     MFMA and Dq_i = dO_i . (P V)_i (stored to a B*H*S workspace); pass 2
@@ -23,6 +24,7 @@
 // diagonal, where a causal forward wrote zeros.
 #include "bwd_bh.h"
 #include "bwd_bh64.h"
+#include "bwd_half.h"
 #include "bwd_tiled.h"
 #include "bwd_wide.h"
 #include "common.h"
@@ -306,13 +308,6 @@ hipError_t launch_dp(const BwdArgs& a, hipStream_t s) {
 
 }  // namespace
 
-// Workgroup shapes of the tiled kernels: query-stationary NQS x NKS,
-// key-stationary NKB x NQS.  4 x 1 for both was best or within 3% of the
-// best of nine shapes on MI355X for the c1 causal, c1 non-causal and c2
-// causal backward; with stored probs, launch_tiled_probs also takes 4 x 2
-// where the grid fills the device's slots better with it.
-constexpr int kBwdQNqs = 4, kBwdQNks = 1, kBwdKvNkb = 4, kBwdKvNqs = 1;
-
 hipError_t bwd_wait_expired(unsigned int* count, bool clear) { return wait_expired_take(count, clear); }
 
 bool bwd_tiled_ok(const BwdArgs& a) {
@@ -322,16 +317,23 @@ bool bwd_tiled_ok(const BwdArgs& a) {
            ((int64_t)(a.S + 64) * a.ts + a.D) * 4 < ((int64_t)1 << 31);
 }
 
-// The one-workgroup-per-(b, h) kernels run a (b, h)'s steps in sequence, so
-// one (b, h) takes 30-80 us whatever the batch.  With causal stored probs (and
-// the D = 32 drop-in) they still beat the query-/key-stationary pair at any
-// batch; rebuilding P from lse, and the D = 64 drop-in, only once the (b, h)
-// pairs fill the CUs (S = 256, H = 8, B = 4: D = 64 from lse 83.2 -> 48.0 us,
-// D = 32 from lse 32.3 -> 27.5 us, D = 64 drop-in 84.4 -> 77.8 us with the
-// pair; B = 32 keeps the per-(b, h) kernels).
-static bool bh_enough(const BwdArgs& a) {
-    if (a.probs && (a.causal || a.D == 32)) return true;
-    return (int64_t)a.B * a.H >= device_cus();
+// The one-workgroup-per-(b, h) kernels (S <= 256, fp32 MFMA, no workspace, each
+// stored P read once) against the query-/key-stationary pair on split operands
+// (P read twice).  The drop-in call keeps them for every shape they took
+// before, since its other kernels need a workspace that it may have to
+// allocate: D = 32, and D = 64 where the (b, h) pairs fill the CUs.  Else, us at
+// H = 8, per-(b, h) against pair:
+//   D = 64 causal stored probs, S = 64: B 2 14.2, 15.9; S = 128: B 2 25.5, 24.0,
+//     B 8 26.3, 26.4, B 32 28.8, 31.7; S = 256: B 2 62, 37, B 8 63, 41, B 32
+//     68, 66 (kept: the same bits as the drop-in there).
+//   D = 32 from lse, forward included, S = 256: B 32 44.0, 46.7, B 64 88.8, 98.4;
+//     S = 128: B 32 26.9, 23.1, B 64 48, 40; with fewer (b, h) than CUs S = 256
+//     B 8 36, 24.
+//   D = 64 from lse: the pair everywhere (S = 256 B 32 105, 90).
+static bool bh_better(const BwdArgs& a) {
+    const bool full = (int64_t)a.B * a.H >= device_cus();
+    if (!a.probs) return a.D == 32 && a.S > 128 && full;
+    return a.D == 32 || full || (a.causal && a.S <= 128);
 }
 
 // The head-dim-split kernels of bwd_wide.h: D % 4 == 0 up to 256, 16-byte
@@ -348,24 +350,26 @@ bool bwd_recompute_ok(const BwdArgs& a) { return a.o && a.lse && (bwd_tiled_ok(a
 
 bool bwd_uses_workspace(const BwdArgs& a) {
     if (!a.probs) return !bwd_tiled_ok(a);  // recompute mode: the wide kernels pass Dq through it
-    return !(bwd_tiled_ok(a) && bh_enough(a) && (bwd::bh_ok(a) || bwd::bh_probs64_ok(a)));
+    return !(bwd_tiled_ok(a) && bh_better(a) && (bwd::bh_ok(a) || bwd::bh_probs64_ok(a)));
 }
 
 hipError_t launch_attn_bwd(const BwdArgs& a, hipStream_t s) {
     // recompute mode (no probs): the tiled kernels, or the wide ones with the Dq workspace
     if (!a.probs && !(bwd_recompute_ok(a) && (bwd_tiled_ok(a) || a.dvec))) return hipErrorInvalidValue;
     if (bwd_tiled_ok(a)) {
-        if (bh_enough(a) && bwd::bh_ok(a)) return bwd::launch_bh(a, s);
-        if (bh_enough(a) && (bwd::bh_probs64_ok(a) || bwd::bh_lse64_ok(a))) return bwd::launch_bh64(a, s);
-        if (a.probs) return a.D == 32 ? bwd::launch_tiled_probs<32>(a, s) : bwd::launch_tiled_probs<64>(a, s);
-        if (a.D == 32)
-            return bwd::launch_tiled<32, kBwdQNqs, kBwdQNks, kBwdKvNkb, kBwdKvNqs>(a, s);
-        return bwd::launch_tiled<64, kBwdQNqs, kBwdQNks, kBwdKvNkb, kBwdKvNqs>(a, s);
+        if (bh_better(a) && bwd::bh_ok(a)) return bwd::launch_bh(a, s);
+        if (bh_better(a) && bwd::bh_probs64_ok(a)) return bwd::launch_bh64(a, s);
+        return a.D == 32 ? bwd::launch_half<32, 4, 1, true>(a, s) : bwd::launch_half<64, 4, 1, true>(a, s);
     }
     if (bwd_wide_ok(a)) {
-        if (a.D <= 32) return bwd::launch_wide<32, 4, 1, 2>(a, s);
-        if (a.D <= 64) return bwd::launch_wide<64, 4, 1, 2>(a, s);
-        if (a.D <= 128) return bwd::launch_wide<128, 4, 2, 2>(a, s);
+        if (a.D <= 32) return bwd::launch_half<32, 4, 1, false>(a, s);
+        if (a.D <= 64) return bwd::launch_half<64, 4, 1, false>(a, s);
+        // 64-row blocks until 128-row ones give every CU one (one 8-wave
+        // workgroup per CU): 8 (b, h) of 1024 rows with stored probs 201 -> 178
+        // us, 32 232 -> 225; with more, 128-row blocks read each tile half as often
+        if (a.D <= 128)
+            return (int64_t)((a.S + 127) / 128) * a.B * a.H <= 256 ? bwd::launch_half<128, 2, 2, false>(a, s)
+                                                                   : bwd::launch_half<128, 4, 2, false>(a, s);
         return bwd::launch_wide<256, 2, 4, 1>(a, s);
     }
     if (a.D <= 32) return launch_dp<32>(a, s);

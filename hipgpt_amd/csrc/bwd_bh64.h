@@ -19,15 +19,6 @@
 // steps t < j and loads no P above the diagonal; every wave's partial-sum
 // and dQ-term slots start at zero, so the fixed-order sums need no masks.
 // All summation orders are fixed: results are deterministic.
-//
-// LSE (probs-free): Dq_i = dO_i . O_i needs no sweep over the keys, so each
-// wave computes it, with lse' = lse log2 e, for the rows of its own query
-// tile into an LDS table before the first step; no partial sums are formed.
-// Each step rebuilds P = exp2(S' - lse') from S' = (c log2 e) Q K^T (K
-// pre-scaled in registers; masks on the causal diagonal and on keys past S
-// only), the S' and dP chains starting from -lse' and -Dq, so P = exp2(S'
-// chain) and dS = P * (dP chain).  160 MFMAs per wave and step; the
-// mid-step barrier only orders the single buffer of dQ terms.
 #pragma once
 
 #include "bwd_bh.h"
@@ -48,18 +39,17 @@ constexpr int PPd = DK + 8;     // pitch of a dQ term's rows: rows q and q+4 on 
 // immediate offsets reach 64 KB only)
 constexpr int XS = 0;                        // per-wave scratch [NW][BK][XP]
 constexpr int RING = XS + NW * BK * XP;
-constexpr int PD = RING + SLOTS * 2 * TILE;  // partial row sums [2][NW][BK]; LSE: lse' and Dq [2][MAXS]
+constexpr int PD = RING + SLOTS * 2 * TILE;  // partial row sums [2][NW][BK]
 constexpr int DQP = PD + 2 * NW * BK;        // dQ terms [NW][BK][PPd]
 constexpr int TOTAL = DQP + NW * BK * PPd;
 constexpr int kLdsBytes = TOTAL * 4;
 constexpr int DQCOL = BK;  // the step's Dq in the scratch rows' pitch padding
 static_assert(XP >= BK + 4, "room for the step's Dq in the scratch pitch");
-static_assert(NW * BK == MAXS, "the LSE mode's lse' and Dq tables fit the partial-sum slots");
 static_assert(kLdsBytes <= 160 * 1024, "LDS of the D = 64 single-read kernel");
 static_assert(BK * CPRd == NW * 64, "one 16-byte chunk of each of Q and dO per thread and tile");
 }  // namespace p64
 
-template <bool CAUSAL, bool LSE>
+template <bool CAUSAL>
 __global__ __launch_bounds__(NW * 64) void bwd_bh64_kernel(BwdArgs a) {
     using namespace p64;
     extern __shared__ __attribute__((aligned(16))) float lds[];
@@ -98,15 +88,14 @@ __global__ __launch_bounds__(NW * 64) void bwd_bh64_kernel(BwdArgs a) {
     };
 
     const __amdgpu_buffer_rsrc_t pr = __builtin_amdgcn_make_buffer_rsrc(
-        LSE ? nullptr : const_cast<float*>(a.probs) + (int64_t)bhi * S * S, 0, LSE ? 0 : S * S * 4, kBufferFlags);
+        const_cast<float*>(a.probs) + (int64_t)bhi * S * S, 0, S * S * 4, kBufferFlags);
 
     // The wave's keys: V (B operand of dP, lane (c, h) holding dims
-    // 32h .. 32h+31 of key kj), with LSE also K pre-scaled by c log2 e (B
-    // operand of S', the same layout), and K as the B operand of the dQ
+    // 32h .. 32h+31 of key kj), and K as the B operand of the dQ
     // product over keys (block n, step s: key dq_key(s, h), dim 32n + c),
     // read back through the scratch.  Only what the first step needs is
     // requested before it.
-    float vr[DK / 2], kq[NB][16], kr[LSE ? DK / 2 : 1];
+    float vr[DK / 2], kq[NB][16];
     floatx16 p, pn;  // stored probs: P of the step's query tile and of the next one
     const Stage r0 = ring_load(0);
     Stage rn = ring_load(1);
@@ -117,39 +106,14 @@ __global__ __launch_bounds__(NW * 64) void bwd_bh64_kernel(BwdArgs a) {
     if (active) {
 #pragma unroll
         for (int s = 0; s < DK / 8; ++s) vv[s] = vl.load(kj, hf * (DK / 8) + s);
-        if (!LSE && meets(0)) load_p_tile(p, pr, 0, kj, kval, hf, S);
+        if (meets(0)) load_p_tile(p, pr, 0, kj, kval, hf, S);
 #pragma unroll
         for (int s = 0; s < DK / 8; ++s) kv[s] = kl.load(kj, hf * (DK / 8) + s);
     }
     ring_store(0, r0);
-    if constexpr (LSE) {
-        // the rows of query tile `wave`: lse' = lse log2 e (+inf past S, so P
-        // = 0 there) and Dq = dO . O, lane (c, h) summing dims 32h .. 32h+31
-        // of row c; tables [S] at PD (lse') and PD + MAXS (Dq)
-        if (active) {
-            RowLoader ol, gl;
-            ol.init(a.o + base, a.ts, S, DK);
-            gl.init(a.go + base, a.ts, S, DK);
-            const int row = wave * BK + c;
-            const float lsev = row < S ? a.lse[(int64_t)bhi * S + row] : 0.f;
-            float d = 0.f;
-#pragma unroll
-            for (int s2 = 0; s2 < DK / 8; ++s2) {
-                const floatx4 o4 = ol.load(row, hf * (DK / 8) + s2), g4 = gl.load(row, hf * (DK / 8) + s2);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) d = fmaf(g4[e], o4[e], d);
-            }
-            d += __shfl_xor(d, 32);
-            if (hf == 0) {
-                lds[PD + row] = row < S ? lsev * kLog2e : kInf;
-                lds[PD + MAXS + row] = d;
-            }
-        }
-    } else {
-        // every wave's partial-sum slots start at zero: waves past the last
-        // key tile, and causally before their diagonal, leave them so
-        lds[PD + (hf * NW + wave) * BK + c] = 0.f;
-    }
+    // every wave's partial-sum slots start at zero: waves past the last
+    // key tile, and causally before their diagonal, leave them so
+    lds[PD + (hf * NW + wave) * BK + c] = 0.f;
     // the same for the dQ-term slots
 #pragma unroll
     for (int k = 0; k < BK * (DK / 4) / 64; ++k) {
@@ -235,9 +199,8 @@ __global__ __launch_bounds__(NW * 64) void bwd_bh64_kernel(BwdArgs a) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 vr[4 * s + j] = vv[s][j];
-                if constexpr (LSE) kr[4 * s + j] = kv[s][j] * (a.scale * kLog2e);
             }
-        if (!LSE && nt > 1 && meets(1)) load_p_tile(pn, pr, 1, kj, kval, hf, S);
+        if (nt > 1 && meets(1)) load_p_tile(pn, pr, 1, kj, kval, hf, S);
         // K through the scratch, one 32-dim block at a time: lanes of half n
         // hold dims 32n .. 32n+31.  The lanes of the other half read what
         // these lanes wrote: a wave's LDS accesses run in order, and the
@@ -304,7 +267,7 @@ __global__ __launch_bounds__(NW * 64) void bwd_bh64_kernel(BwdArgs a) {
     // Step t (t % 2 == PAR) of every wave.  Stored probs: pc holds P of tile
     // t, the other buffer P of tile t+1 (requested a step ago); P of tile t+2
     // goes into pc once dS is formed, so the two buffers alternate roles and
-    // nothing is copied.  LSE: P is rebuilt, pc unused.
+    // nothing is copied.
     auto step = [&](auto par_tag, int t, floatx16& pc) {
         constexpr int PAR = decltype(par_tag)::value;
         const bool cur = meets(t);
@@ -312,97 +275,60 @@ __global__ __launch_bounds__(NW * 64) void bwd_bh64_kernel(BwdArgs a) {
         const float* gt = qt + TILE;
         // the dQ rows of tile t-1 (its terms were published by the last barrier)
         if (t > 0) reduce_dq(t - 1);
-        if constexpr (LSE) {
-            lds_barrier();  // every wave has read the dQ terms of tile t-1
-            if (cur) {
-                // S' - lse' and dP - Dq, register r <-> query t*32 + acc_key(r, h), lane <-> key
-                floatx16 sc, dpc;
+        // dP of tile t and its partial row sums
+        floatx16 dp;
+        if (cur) {
+            dp = dp_tile(gt);
+            partial(std::integral_constant<int, PAR>{}, pc, dp);
+        }
+        lds_barrier();  // the partial sums of tile t; every wave has read the dQ terms of tile t-1
+        if (cur) {
+            // Dq of query tile t (lane: query c): the partials in key-tile
+            // order, kept in the scratch's padding for the register-order reads
+            float dsum = 0.f;
 #pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const floatx4 l4 = *reinterpret_cast<const floatx4*>(lds + PD + t * BK + 8 * g + 4 * hf);
-                    const floatx4 d4 = *reinterpret_cast<const floatx4*>(lds + PD + MAXS + t * BK + 8 * g + 4 * hf);
+            for (int v = 0; v < NW; ++v) dsum += pdl[(PAR * NW + v) * BK];
+            if (hf == 0) X[(c >> 2) * XP + DQCOL + (c & 3)] = dsum;
+            asm volatile("" ::: "memory");
+            // (written out here: through grad_v and grad_kq this branch
+            // spills two registers at 256 VGPRs)
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        sc[4 * g + j] = -l4[j];
-                        dpc[4 * g + j] = -d4[j];
-                    }
-                }
-                sc = chain(qt, kr, sc);
-                dpc = chain(gt, vr, dpc);
-                floatx16 pv, ds;
-                if (kedge || (CAUSAL && t == wave)) {  // keys past S, the causal diagonal
+            for (int n = 0; n < NB; ++n)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const bool vis = kval && (!CAUSAL || kj <= t * BK + acc_key(r, hf));
-                        pv[r] = vis ? fast_exp2(sc[r]) : 0.f;
-                        ds[r] = pv[r] * dpc[r];
-                    }
-                } else {
+                for (int r = 0; r < 16; ++r)
+                    accv[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(gt[acc_key(r, hf) * RPd + 32 * n + c], pc[r],
+                                                                   accv[n], 0, 0, 0);
+            floatx16 ds;
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        pv[r] = fast_exp2(sc[r]);
-                        ds[r] = pv[r] * dpc[r];
-                    }
-                }
-                grad_v(gt, pv);
-                grad_kq(qt, ds);
+            for (int g = 0; g < 4; ++g) {
+                const floatx4 d4 = *reinterpret_cast<const floatx4*>(X + (2 * g + hf) * XP + DQCOL);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) ds[4 * g + j] = pc[4 * g + j] * (dp[4 * g + j] - d4[j]);
             }
-        } else {
-            // dP of tile t and its partial row sums
-            floatx16 dp;
-            if (cur) {
-                dp = dp_tile(gt);
-                partial(std::integral_constant<int, PAR>{}, pc, dp);
+            if (t + 2 < nt) load_p_tile(pc, pr, t + 2, kj, kval, hf, S);
+#pragma unroll
+            for (int n = 0; n < NB; ++n)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    acck[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(qt[acc_key(r, hf) * RPd + 32 * n + c], ds[r],
+                                                                   acck[n], 0, 0, 0);
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                *reinterpret_cast<floatx4*>(X + c * XP + 8 * g + 4 * hf) =
+                    floatx4{ds[4 * g], ds[4 * g + 1], ds[4 * g + 2], ds[4 * g + 3]};
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int n = 0; n < NB; ++n) {
+                floatx16 aq =
+                    __builtin_amdgcn_mfma_f32_32x32x2f32(X[dq_key(0, hf) * XP + c], kq[n][0], floatx16{}, 0, 0, 0);
+#pragma unroll
+                for (int s = 1; s < 16; ++s)
+                    aq = __builtin_amdgcn_mfma_f32_32x32x2f32(X[dq_key(s, hf) * XP + c], kq[n][s], aq, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) dqw[(8 * (r >> 2) + (r & 3)) * PPd + 32 * n] = aq[r];
             }
-            lds_barrier();  // the partial sums of tile t; every wave has read the dQ terms of tile t-1
-            if (cur) {
-                // Dq of query tile t (lane: query c): the partials in key-tile
-                // order, kept in the scratch's padding for the register-order reads
-                float dsum = 0.f;
-#pragma unroll
-                for (int v = 0; v < NW; ++v) dsum += pdl[(PAR * NW + v) * BK];
-                if (hf == 0) X[(c >> 2) * XP + DQCOL + (c & 3)] = dsum;
-                asm volatile("" ::: "memory");
-                // (written out here: through grad_v and grad_kq this branch
-                // spills two registers at 256 VGPRs)
-#pragma unroll
-                for (int n = 0; n < NB; ++n)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        accv[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(gt[acc_key(r, hf) * RPd + 32 * n + c], pc[r],
-                                                                       accv[n], 0, 0, 0);
-                floatx16 ds;
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const floatx4 d4 = *reinterpret_cast<const floatx4*>(X + (2 * g + hf) * XP + DQCOL);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) ds[4 * g + j] = pc[4 * g + j] * (dp[4 * g + j] - d4[j]);
-                }
-                if (t + 2 < nt) load_p_tile(pc, pr, t + 2, kj, kval, hf, S);
-#pragma unroll
-                for (int n = 0; n < NB; ++n)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        acck[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(qt[acc_key(r, hf) * RPd + 32 * n + c], ds[r],
-                                                                       acck[n], 0, 0, 0);
-#pragma unroll
-                for (int g = 0; g < 4; ++g)
-                    *reinterpret_cast<floatx4*>(X + c * XP + 8 * g + 4 * hf) =
-                        floatx4{ds[4 * g], ds[4 * g + 1], ds[4 * g + 2], ds[4 * g + 3]};
-                asm volatile("" ::: "memory");
-#pragma unroll
-                for (int n = 0; n < NB; ++n) {
-                    floatx16 aq =
-                        __builtin_amdgcn_mfma_f32_32x32x2f32(X[dq_key(0, hf) * XP + c], kq[n][0], floatx16{}, 0, 0, 0);
-#pragma unroll
-                    for (int s = 1; s < 16; ++s)
-                        aq = __builtin_amdgcn_mfma_f32_32x32x2f32(X[dq_key(s, hf) * XP + c], kq[n][s], aq, 0, 0, 0);
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) dqw[(8 * (r >> 2) + (r & 3)) * PPd + 32 * n] = aq[r];
-                }
-            } else if (t + 2 < nt && meets(t + 2)) {
-                load_p_tile(pc, pr, t + 2, kj, kval, hf, S);  // causally: the wave's first tile
-            }
+        } else if (t + 2 < nt && meets(t + 2)) {
+            load_p_tile(pc, pr, t + 2, kj, kval, hf, S);  // causally: the wave's first tile
         }
         ring_store(t + 1, rn);
         rn = ring_load(t + 2);
@@ -435,20 +361,17 @@ __global__ __launch_bounds__(NW * 64) void bwd_bh64_kernel(BwdArgs a) {
 
 // D = 64 (causal or not), S <= 256, and the tiled kernels' layout conditions
 // (checked by the caller).  Stored probs are read as single floats, so there
-// is no condition on S or on the probs' alignment; without them the forward's
-// O and lse are required (the caller checks that too).
+// is no condition on S or on the probs' alignment.
 inline bool bh_probs64_ok(const BwdArgs& a) {
     return a.probs && a.D == bh::p64::DK && a.S >= 1 && a.S <= bh::MAXS;
 }
-inline bool bh_lse64_ok(const BwdArgs& a) { return !a.probs && a.D == bh::p64::DK && a.S >= 1 && a.S <= bh::MAXS; }
 
 inline hipError_t launch_bh64(const BwdArgs& a, hipStream_t s) {
     const int64_t grid = (int64_t)a.B * a.H;
     if (grid <= 0 || grid > 0x7fffffff) return hipErrorInvalidConfiguration;
-    const int mode = (a.causal ? 1 : 0) + (a.probs ? 0 : 2);
-    static void (*const kerns[4])(BwdArgs) = {bh::bwd_bh64_kernel<false, false>, bh::bwd_bh64_kernel<true, false>,
-                                              bh::bwd_bh64_kernel<false, true>, bh::bwd_bh64_kernel<true, true>};
-    static std::atomic<unsigned long long> attr_set[4] = {{0}, {0}, {0}, {0}};
+    const int mode = a.causal ? 1 : 0;
+    static void (*const kerns[2])(BwdArgs) = {bh::bwd_bh64_kernel<false>, bh::bwd_bh64_kernel<true>};
+    static std::atomic<unsigned long long> attr_set[2] = {{0}, {0}};
     hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(kerns[mode]), bh::p64::kLdsBytes, attr_set[mode]);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kerns[mode], dim3((unsigned)grid), dim3(bh::NW * 64), bh::p64::kLdsBytes, s, a);

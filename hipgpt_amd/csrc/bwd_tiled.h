@@ -1,17 +1,18 @@
 // bwd_tiled.h -- LDS-tiled MFMA kernels of the attention backward on the
 // forward's probabilities (HipGPT src/hip_kernels.cpp:1159-1272), for head
-// dims 32 and 64 with 16-byte aligned rows.
+// dims 32 and 64 with 16-byte aligned rows.  The workgroups of bwd_half.h run
+// them where their split operands do not hold the data.
 //
 // Math per (b, h), scale c = 1/sqrt(D):
 //   dP = dO V^T,  Dq_i = sum_j P_ij dP_ij,  dS = P o (dP - Dq),
 //   dQ = c dS K,  dK = c dS^T Q,  dV = P^T dO.
 // Two kernels, every gradient element written once (no atomics, no memset):
-//   * bwd_q_kernel (query-stationary): wave (qs, ks) owns 32 queries and every
+//   * BwdQ (query-stationary): wave (qs, ks) owns 32 queries and every
 //     NKS-th key tile.  One pass over the keys accumulates
 //       A = (P o dP) K,  Bm = P K,  Dq = rowsum(P o dP),
 //     and dQ = c (A - Dq Bm), so P and V are read once; the key splits are
 //     summed through LDS.  Dq goes to the workspace for the second kernel.
-//   * bwd_kv_kernel (key-stationary): wave (ks, qs) owns 32 keys (V in
+//   * BwdKV (key-stationary): wave (ks, qs) owns 32 keys (V in
 //     registers) and every NQS-th query tile; dP = dO V^T lands with one key
 //     per lane and the queries in the accumulator's register order, which is
 //     the B-operand layout of dV^T += dO^T P and dK^T += Q^T dS, so P and dS
@@ -31,9 +32,8 @@
 // forms it from the dO rows it loads; the query-stationary one then forms
 // dQ = c dS K directly) and P is rebuilt per tile as exp2(S' - lse'),
 // S' = (c log2 e) q.k from the operand tiles already in LDS plus a row-major K
-// (resp. Q) tile, with the causal mask applied on the diagonal tiles.  As
-// neither kernel then reads the other's output, bwd_pair_kernel runs both
-// kinds of workgroup in one launch.
+// (resp. Q) tile, with the causal mask applied on the diagonal tiles.  Neither
+// kernel then reads the other's output.
 #pragma once
 
 #include <type_traits>
@@ -607,113 +607,6 @@ struct BwdKV {
         }
     }
 };
-
-template <int DP, int NQS, int NKS, bool CAUSAL, bool RECOMP>
-__global__ __launch_bounds__(NQS* NKS * 64) void bwd_q_kernel(BwdArgs a, int nqb) {
-    using K = BwdQ<DP, NQS, NKS, CAUSAL, RECOMP>;
-    __shared__ __attribute__((aligned(16))) float lds[K::LDS_FLOATS];
-    __shared__ int simd_slots[NQS * NKS];
-    const int BH = a.B * a.H;
-    K::run(a, lds, simd_slots, nqb, blockIdx.x % BH, blockIdx.x / BH);
-}
-
-template <int DP, int NKB, int NQS, bool CAUSAL, bool RECOMP>
-__global__ __launch_bounds__(NKB* NQS * 64) void bwd_kv_kernel(BwdArgs a, int nkb) {
-    using K = BwdKV<DP, NKB, NQS, CAUSAL, RECOMP>;
-    __shared__ __attribute__((aligned(16))) float lds[K::LDS_FLOATS];
-    __shared__ int simd_slots[NKB * NQS];
-    const int BH = a.B * a.H;
-    K::run(a, lds, simd_slots, nkb, blockIdx.x % BH, blockIdx.x / BH);
-}
-
-// Recompute mode: the query- and key-stationary workgroups of the same shape
-// in one grid, dealt in chunks of B*H workgroups as query rank 0, key rank 0,
-// query rank 1, ... (the heaviest causal blocks of each kind first), so that
-// both kinds share the CUs -- twice the waves in flight of either kernel
-// alone -- and the pair costs one launch.
-template <int DP, int NQS, int NKS, int NKB, int NQS2, bool CAUSAL>
-__global__ __launch_bounds__(NQS* NKS * 64) void bwd_pair_kernel(BwdArgs a, int nr) {
-    using KQ = BwdQ<DP, NQS, NKS, CAUSAL, true>;
-    using KK = BwdKV<DP, NKB, NQS2, CAUSAL, true>;
-    static_assert(NQS * NKS == NKB * NQS2 && NQS == NKB, "both kinds need the same workgroup and block counts");
-    constexpr int LF = KQ::LDS_FLOATS > KK::LDS_FLOATS ? KQ::LDS_FLOATS : KK::LDS_FLOATS;
-    __shared__ __attribute__((aligned(16))) float lds[LF];
-    __shared__ int simd_slots[NQS * NKS];
-    const int BH = a.B * a.H;
-    const int chunk = blockIdx.x / BH, bh = blockIdx.x % BH;
-    if (chunk & 1)
-        KK::run(a, lds, simd_slots, nr, bh, chunk >> 1);
-    else
-        KQ::run(a, lds, simd_slots, nr, bh, chunk >> 1);
-}
-
-// Both kernels for one problem: stored probs, two launches (the second reads
-// the first's Dq); recompute mode, one launch of the pair kernel.
-template <int DP, int QNQS, int QNKS, int KNKB, int KNQS, bool CAUSAL, bool RECOMP>
-hipError_t launch_tiled_mode(const BwdArgs& a, hipStream_t s) {
-    const int BH = a.B * a.H;
-    const int nqb = (a.S + QNQS * BK - 1) / (QNQS * BK);
-    const int nkb = (a.S + KNKB * BK - 1) / (KNKB * BK);
-    const int64_t g1 = (int64_t)nqb * BH, g2 = (int64_t)nkb * BH;
-    if (g1 <= 0 || g1 + g2 > 0x7fffffff) return hipErrorInvalidConfiguration;
-    if constexpr (RECOMP) {
-        hipLaunchKernelGGL((bwd_pair_kernel<DP, QNQS, QNKS, KNKB, KNQS, CAUSAL>), dim3((unsigned)(g1 + g2)),
-                           dim3(QNQS * QNKS * 64), 0, s, a, nqb);
-        return hipGetLastError();
-    } else {
-        hipLaunchKernelGGL((bwd_q_kernel<DP, QNQS, QNKS, CAUSAL, false>), dim3((unsigned)g1), dim3(QNQS * QNKS * 64), 0,
-                           s, a, nqb);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL((bwd_kv_kernel<DP, KNKB, KNQS, CAUSAL, false>), dim3((unsigned)g2), dim3(KNKB * KNQS * 64),
-                           0, s, a, nkb);
-        return hipGetLastError();
-    }
-}
-
-// Stored probs: 4 x 1 workgroups, or 4 x 2 -- each query-stationary
-// workgroup's keys and each key-stationary workgroup's queries split over two
-// more waves, so a workgroup takes about half as long at half as many resident
-// slots (one 8-wave workgroup per CU instead of two 4-wave ones; the same
-// 128-row blocks, so the same grid).  The split pays when the 4 x 1 grid
-// would end on a partly filled round: without a causal mask, when
-// ceil(G / S2) / 2 (+10% for the wider workgroup) is below ceil(G / S1);
-// causally (longest blocks first), when the whole grid fits one 4 x 2 round.
-// Cache-rotated, D = 64: the HipGPT drop-in at B8 H12 S1024 (G = 768) 868 ->
-// 737 us, B8 H8 S512 non-causal (G = 256) 148 -> 135, causal 142 -> 131;
-// kept 4 x 1: non-causal B2 H12 S2048 (G = 384: 856 against 940 us), D = 32
-// B8 H8 S1024 (G = 512: 259 against 285), causal B8 H12 S1024 (G = 768: 410
-// against 436).  The probs-free pair keeps 4 x 1 (449 against 482 us at B8
-// H12 S1024 causal).
-template <int DP>
-hipError_t launch_tiled_probs(const BwdArgs& a, hipStream_t s) {
-    static ResidentSlots c1[2], c2[2];
-    const int ci = a.causal ? 1 : 0;
-    const void* k1 = a.causal ? reinterpret_cast<const void*>(bwd_q_kernel<DP, 4, 1, true, false>)
-                              : reinterpret_cast<const void*>(bwd_q_kernel<DP, 4, 1, false, false>);
-    const void* k2 = a.causal ? reinterpret_cast<const void*>(bwd_q_kernel<DP, 4, 2, true, false>)
-                              : reinterpret_cast<const void*>(bwd_q_kernel<DP, 4, 2, false, false>);
-    const int64_t S1 = c1[ci].get(k1, 4 * 64, 0), S2 = c2[ci].get(k2, 8 * 64, 0);
-    const int64_t G = (int64_t)((a.S + 4 * BK - 1) / (4 * BK)) * a.B * a.H;
-    bool split = false;
-    if (S1 > 0 && S2 > 0)
-        split = a.causal ? G <= S2 : 11 * ((G + S2 - 1) / S2) < 20 * ((G + S1 - 1) / S1);
-    if (split)
-        return a.causal ? launch_tiled_mode<DP, 4, 2, 4, 2, true, false>(a, s)
-                        : launch_tiled_mode<DP, 4, 2, 4, 2, false, false>(a, s);
-    return a.causal ? launch_tiled_mode<DP, 4, 1, 4, 1, true, false>(a, s)
-                    : launch_tiled_mode<DP, 4, 1, 4, 1, false, false>(a, s);
-}
-
-template <int DP, int QNQS, int QNKS, int KNKB, int KNQS>
-hipError_t launch_tiled(const BwdArgs& a, hipStream_t s) {
-    const bool recomp = a.probs == nullptr;
-    if (a.causal)
-        return recomp ? launch_tiled_mode<DP, QNQS, QNKS, KNKB, KNQS, true, true>(a, s)
-                      : launch_tiled_mode<DP, QNQS, QNKS, KNKB, KNQS, true, false>(a, s);
-    return recomp ? launch_tiled_mode<DP, QNQS, QNKS, KNKB, KNQS, false, true>(a, s)
-                  : launch_tiled_mode<DP, QNQS, QNKS, KNKB, KNQS, false, false>(a, s);
-}
 
 }  // namespace bwd
 }  // namespace hipgpt

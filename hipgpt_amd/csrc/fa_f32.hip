@@ -157,9 +157,6 @@ struct F32Traits {
     }
 };
 
-typedef short v4i16 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
-
 // The products on operands split into two fp16 terms (split.h), the traits
 // every problem runs unless its data need F32Traits (`exact`).  Tiles are two
 // row-major planes; operand layouts as in fa_bf16.hip (v_mfma_f32_32x32x16).
@@ -285,28 +282,13 @@ struct F32HalfTraits {
         const unsigned short* p = Vt + (16 * s + 4 * hf + (r >> 2)) * VRP + db * 32 + (c & 16) + 4 * (r & 3);
         Half8 v;
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(p + t * VPL)));
-            const uint2 hi = __builtin_bit_cast(
-                uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(p + t * VPL + 8 * VRP)));
-            v.t[t] = __builtin_bit_cast(halfx8, uint4{lo.x, lo.y, hi.x, hi.y});
-        }
+        for (int t = 0; t < 2; ++t) v.t[t] = read_rows_tr(p + t * VPL, 8 * VRP);
         return v;
     }
-    struct PReg {
-        Half8 s[2];
-    };
+    using PReg = HalfP;
     template <bool SCALED = false>
     __device__ __forceinline__ static PReg to_p(const floatx16& p) {
-        PReg pb;
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            float x[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) x[j] = p[8 * s + j];
-            pb.s[s] = half8<SCALED>(x, fa::kHalfPScale);
-        }
-        return pb;
+        return half_p<SCALED>(p, fa::kHalfPScale);
     }
     __device__ __forceinline__ static void pv(const VReg& vr, const PReg& pb, floatx16* o, int c, int hf) {
 #pragma unroll

@@ -346,22 +346,6 @@ struct HalfCfg : Cfg<BM, BN, WM, WN, 32> {
     static constexpr int BYTES = 2 * STAGE16 * 2 + SCALES * 4;
 };
 
-// Power of two that brings a magnitude to [2^7, 2^8), and its inverse
-// (magnitudes below 2^-87 as if at 2^-87).
-__device__ __forceinline__ unsigned scale_exp(float m) {
-    const unsigned e = __float_as_uint(m) >> 23;
-    return e < 40u ? 40u : e > 254u ? 254u : e;
-}
-__device__ __forceinline__ float scale_of(unsigned e) { return __uint_as_float((261u - e) << 23); }
-__device__ __forceinline__ float unscale_of(unsigned e) { return __uint_as_float((e - 7u) << 23); }
-
-__device__ __forceinline__ float max4(const floatx4& v) {
-    return fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
-}
-
-typedef short v4i16 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
-
 // The tile on split operands (split.h).  Every row of A and every column of W
 // carries a power of two of its own, from its largest magnitude in the first
 // k-tile (if that is zero there, in the first one where it is not); the
@@ -543,10 +527,7 @@ __device__ __forceinline__ bool gemm_half_tile(const GemmArgs& g, unsigned char*
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
                     const u16* p = Ws + t * C::WPL + s * 16 * C::WP + i * 32;
-                    const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)p));
-                    const uint2 hi = __builtin_bit_cast(
-                        uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(p + 8 * C::WP)));
-                    w[i].t[t] = __builtin_bit_cast(halfx8, uint4{lo.x, lo.y, hi.x, hi.y});
+                    w[i].t[t] = read_rows_tr(p, 8 * C::WP);
                 }
 #pragma unroll
             for (int i = 0; i < C::NB; ++i)

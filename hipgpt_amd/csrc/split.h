@@ -80,4 +80,49 @@ __device__ __forceinline__ floatx16 mfma_half(const Half8& a, const Half8& b, fl
     return mfma_f16(a.t[0], b.t[0], mfma_half_small(a, b, acc));
 }
 
+// Power of two that brings a magnitude to [2^7, 2^8), and its inverse
+// (magnitudes below 2^-87 as if at 2^-87).
+__device__ __forceinline__ unsigned scale_exp(float m) {
+    const unsigned e = __float_as_uint(m) >> 23;
+    return e < 40u ? 40u : e > 254u ? 254u : e;
+}
+__device__ __forceinline__ float scale_of(unsigned e) { return __uint_as_float((261u - e) << 23); }
+__device__ __forceinline__ float unscale_of(unsigned e) { return __uint_as_float((e - 7u) << 23); }
+
+__device__ __forceinline__ float max4(const floatx4& v) {
+    return fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+}
+
+typedef short v4i16 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
+
+// Operand that contracts over the rows of a row-major LDS tile of 16-bit
+// values: column `lane & 15` of the 16 columns the lane's group of 16 points
+// at, four rows from its first one and four from eight rows on (rows8: 16-bit
+// elements from a row to the eighth after it).  Within the group lane r passes
+// the address of row r / 4, columns 4 (r % 4) ..; see fa_bf16.hip.
+__device__ __forceinline__ halfx8 read_rows_tr(const unsigned short* p, int rows8) {
+    const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)p));
+    const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(p + rows8)));
+    return __builtin_bit_cast(halfx8, uint4{lo.x, lo.y, hi.x, hi.y});
+}
+
+// 16 values in accumulator register order as the operand that contracts over
+// them, times s if SCALED.
+struct HalfP {
+    Half8 s[2];
+};
+template <bool SCALED>
+__device__ __forceinline__ HalfP half_p(const floatx16& p, float s) {
+    HalfP h;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        float x[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = p[8 * i + j];
+        h.s[i] = half8<SCALED>(x, s);
+    }
+    return h;
+}
+
 }  // namespace hipgpt
