@@ -510,10 +510,9 @@ int hipgpt_attn_decode_kvcache(const float* q, const float* k_new, const float* 
 
 int hipgpt_attn_wait_expired(unsigned int* count, int clear) {
     if (!count) return HIPGPT_ERR_INVALID;
-    unsigned int fwd = 0, bwd = 0;
-    if (hipgpt::fa_f32_wait_expired(&fwd, clear != 0) != hipSuccess) return HIPGPT_ERR_LAUNCH;
-    if (hipgpt::bwd_wait_expired(&bwd, clear != 0) != hipSuccess) return HIPGPT_ERR_LAUNCH;
-    *count = fwd + bwd;
+    unsigned int n = 0;
+    if (hipgpt::bwd_wait_expired(&n, clear != 0) != hipSuccess) return HIPGPT_ERR_LAUNCH;
+    *count = n;
     return HIPGPT_OK;
 }
 

@@ -110,7 +110,7 @@ struct F32Traits {
     // V^T operands of a tile: lane (c, hf) of block db needs
     // V[acc_key(t, hf)][db*32 + c], t = 0..15 -- four ds_read_b128 per block.
     // VPRE: read before the softmax (VReg holds them) -- the streaming kernel
-    // at DP = 32 and the resident kernel; otherwise each block is read just
+    // at DP = 32; otherwise each block is read just
     // before use.  That brings the streaming kernel at DP = 64 to 128 VGPRs:
     // with WAVES_PER_EU = 4 two 8-wave workgroups share a CU (c3: 132 -> 128
     // us; prefetching V under the same cap spills).
@@ -340,8 +340,6 @@ hipError_t launch_guarded(const AttnArgs& a, bool causal, bool probs, int64_t n1
 }
 
 }  // namespace
-
-hipError_t fa_f32_wait_expired(unsigned int* count, bool clear) { return wait_expired_take(count, clear); }
 
 int fa_f32_padded_dim(int D) {
     if (D <= 32) return 32;

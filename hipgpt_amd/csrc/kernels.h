@@ -26,10 +26,9 @@ hipError_t launch_fa_wide(const AttnArgs& a, bool causal, hipStream_t stream);
 // Any head dim, fp32: one wave per query row (the path for other D > 128).
 hipError_t launch_attn_generic_f32(const AttnArgs& a, bool causal, hipStream_t stream);
 
-// Expired bounded waits (note_wait_expired) of the kernels in fa_f32.hip (the
-// resident-K/V forward) and bwd.hip (the per-(b, h) backward) on the current
-// device; cleared after the read when `clear` is set.
-hipError_t fa_f32_wait_expired(unsigned int* count, bool clear);
+// Expired bounded waits (note_wait_expired) of the kernels in bwd.hip (the
+// per-(b, h) backward) on the current device; cleared after the read when
+// `clear` is set.
 hipError_t bwd_wait_expired(unsigned int* count, bool clear);
 
 // KV-cache decode step: the cache is a.k / a.v (with a.k_* / a.v_* strides,

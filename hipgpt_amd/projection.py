@@ -3,7 +3,7 @@
 The QKV projection and the output projection around the attention
 (``src/transformer_layer.cpp:217``, ``:220``) are ``launch_matmul_add_bias``
 calls (``include/hip_kernels.h:7``, ``src/hip_kernels.cpp:113-154``).  Every
-call goes through the C ABI to the fp32 MFMA GEMM; torch only provides
+call goes through the C ABI to the fp32 GEMM; torch only provides
 device memory and streams.
 
 * :func:`launch_matmul_add_bias`, :func:`launch_matmul` -- the reference's
@@ -49,7 +49,7 @@ def launch_matmul(A, B, C, M, N, K):
 
 def gemm_bias(A, W, bias=None, out=None, out_dtype=torch.float32, seg_w=None, seg_stride=0, ldc=None,
               stream=None):
-    """``A [M, K] @ W [K, N] (+ bias [N])`` on fp32 MFMA.
+    """``A [M, K] @ W [K, N] (+ bias [N])`` in fp32.
 
     A and W are 2-D float32 tensors with unit column stride (any row stride).
     Output column ``n`` is stored at ``out + (n // seg_w) * seg_stride + m * ldc
