@@ -15,18 +15,19 @@
 // Tiling: a workgroup owns a BM x BN tile of C and walks K in steps of 32.
 // Each wave computes a WM x WN sub-tile as C^T = W^T A^T, so an accumulator
 // register group holds four consecutive output columns of one row (16-byte
-// stores, 16-byte bias loads).  Operand staging: global -> registers -> LDS,
-// double buffered, one barrier per k-tile; the next tile's global loads are in
-// flight during the MFMAs.
+// stores, 16-byte bias loads).  Operand staging: global -> registers -> LDS; the
+// next tile's global loads are in flight during the MFMAs.
 //
-// gemm_half_tile runs every problem with 16-byte rows on operands split into
-// two fp16 terms (split.h; v_mfma_f32_32x32x16_f16, three per product): M 8192
-// N 2304 K 768 222 -> 120 us, M 8192 N 768 K 256 30 -> 22.5; error against 64
-// bits 4.9e-7 -> 3.1e-7 and 2.9e-7 -> 2.1e-7.  The matrix cores are busy 40% of
-// the time, the LDS 57%, the vector ALUs 33% (the split).
+// gemm_terms_tile runs every problem with 16-byte rows on operands split into
+// three bf16 terms (terms.h; v_mfma_f32_32x32x16_bf16, six per product).  Against
+// the fp32 tile, us, and error against 64 bits: M 8192 N 2304 K 768 227 -> 174,
+// 3.5e-7 -> 3.0e-7; M 8192 N 768 K 256 30.0 -> 27.9, 2.0e-7 -> 1.7e-7; M 1024 N
+// 768 K 256 13.2 -> 10.7.  Bound by the matrix cores and, in turn with them, the
+// conversion of the next k-tile: six MFMAs per product at 174 us are 1.0
+// PFLOP/s, of the 1.62 that bf16 MFMAs alone reach on random data.
 //
-// gemm_f32_tile (v_mfma_f32_32x32x2_f32) takes tiles whose data the split does
-// not hold and operands without 16-byte rows:
+// gemm_f32_tile (v_mfma_f32_32x32x2_f32) takes tiles with a result that is not
+// finite on the terms, and operands without 16-byte rows:
 //   A tile [BM][GBK] (pitch GBK+4 floats): lane (c, h) reads row c,
 //     k = (GBK/2)h + s as ds_read_b128 (four k-steps per read).
 //   W tile [GBK][BN] (pitch BN+4, second half of the k rows shifted by 32
@@ -38,7 +39,7 @@
 // k = (GBK/2)h + s at step s, the same bijection for both operands.
 #include "common.h"
 #include "kernels.h"
-#include "split.h"
+#include "terms.h"
 
 namespace hipgpt {
 
@@ -334,32 +335,28 @@ __device__ __forceinline__ void gemm_f32_tile(const GemmArgs& g, float* lds) {
     store_tile<C, VEC, BF16OUT>(g, acc, lds, m0 + wm0, n0 + wn0, wave, lane);
 }
 
-// LDS of the split-operand tile (bytes of one stage): two planes (terms) of
-// the A tile [BM][32], pitch 40, each row's k in MFMA operand order, and two
-// of the W tile [32][BN], row-major, pitch BN + 16.
+// LDS of the tile on bf16 terms (one stage): three planes (terms) of the A tile
+// [BM][32], pitch 40, each row's k in MFMA operand order, and three of the W
+// tile [32][BN], row-major, pitch BN + 16.
 template <int BM, int BN, int WM, int WN>
-struct HalfCfg : Cfg<BM, BN, WM, WN, 32> {
+struct TermCfg : Cfg<BM, BN, WM, WN, 32> {
     static constexpr int AP = 40, WP = BN + 16;
     static constexpr int APL = BM * AP, WPL = 32 * WP;
-    static constexpr int STAGE16 = 2 * (APL + WPL);  // 16-bit elements of a stage
-    static constexpr int SCALES = BM + BN + (BM / WM) * (BN / WN) * BN;  // floats: 1 / row and column scales, column maxima
-    static constexpr int BYTES = 2 * STAGE16 * 2 + SCALES * 4;
+    static constexpr int STAGE16 = 3 * (APL + WPL);  // 16-bit elements
+    static constexpr int BYTES = STAGE16 * 2 + 16;   // and the not-finite flag
 };
 
-// The tile on split operands (split.h).  Every row of A and every column of W
-// carries a power of two of its own, from its largest magnitude in the first
-// k-tile (if that is zero there, in the first one where it is not); the
-// accumulators are divided by both at the end.  A value more than 255 times
-// that magnitude overflows and the result is not finite: false, and the caller
-// runs the fp32 tile.
+// The tile on operands split into three bf16 terms (terms.h).  One LDS stage:
+// the next k-tile waits in registers while this one is multiplied, and two or
+// three workgroups share a CU, one multiplying while another converts.  False,
+// with nothing stored, where a result is not finite; the caller then runs the
+// fp32 tile.
 template <int BM, int BN, int WM, int WN, bool BF16OUT, bool KF>
-__device__ __forceinline__ bool gemm_half_tile(const GemmArgs& g, unsigned char* lds_raw) {
-    using C = HalfCfg<BM, BN, WM, WN>;
+__device__ __forceinline__ bool gemm_terms_tile(const GemmArgs& g, unsigned char* lds_raw) {
+    using C = TermCfg<BM, BN, WM, WN>;
     typedef unsigned short u16;
     u16* const lds = reinterpret_cast<u16*>(lds_raw);
-    float* const s_row = reinterpret_cast<float*>(lds_raw + 2 * C::STAGE16 * 2);
-    float* const s_col = s_row + BM;
-    float* const s_max = s_col + BN;
+    int* const flag = reinterpret_cast<int*>(lds_raw + C::STAGE16 * 2);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int c = lane & 31, h = lane >> 5;
     const int tiles_n = (g.N + BN - 1) / BN;
@@ -385,7 +382,7 @@ __device__ __forceinline__ bool gemm_half_tile(const GemmArgs& g, unsigned char*
         woff[i] = (int)(((tid / (BN / 4) + i * (C::NT / (BN / 4))) * g.ldw + (nc >= cols ? 0 : nc)) * 4);
     // rows past M and k rows past K read as zero; a row's k past K is masked
     // (it would read the next row)
-    auto load_a = [&](int kt) {
+    auto load = [&](int kt) {
 #pragma unroll
         for (int i = 0; i < C::A_PER; ++i) {
             const floatx4 v =
@@ -393,114 +390,22 @@ __device__ __forceinline__ bool gemm_half_tile(const GemmArgs& g, unsigned char*
                    : __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(ars, aoff[i] + kt * 128, 0, 0));
             ar[i] = KF || kt * 32 + kc < K ? v : zero4();
         }
-    };
-    auto load_w = [&](int kt) {
         const int off = (int)((int64_t)kt * 32 * g.ldw * 4);
 #pragma unroll
         for (int i = 0; i < C::W_PER; ++i)
             wr[i] = KF ? __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(wrs, woff[i], off, 0))
                        : __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(wrs, woff[i] + off, 0, 0));
     };
-
-    // ---- scales ----
-    float sa[C::A_PER];
-    floatx4 sw;
-    load_a(0);
-    load_w(0);
-    {
-        float mx[C::A_PER];
-#pragma unroll
-        for (int i = 0; i < C::A_PER; ++i) mx[i] = 0.f;
-        for (int kt = 0;;) {
-            bool zero = false;
-#pragma unroll
-            for (int i = 0; i < C::A_PER; ++i) {
-                float m = max4(ar[i]);
-#pragma unroll
-                for (int x = 1; x < 8; x <<= 1) m = fmaxf(m, __shfl_xor(m, x));
-                if (mx[i] == 0.f) mx[i] = m;
-                zero |= mx[i] == 0.f && tid / 8 + i * (C::NT / 8) < rows;
-            }
-            if (!__any(zero) || ++kt >= nkt) {
-                if (kt > 0) load_a(0);
-                break;
-            }
-            load_a(kt);
-        }
-#pragma unroll
-        for (int i = 0; i < C::A_PER; ++i) {
-            const unsigned e = scale_exp(mx[i]);
-            sa[i] = scale_of(e);
-            if ((tid & 7) == 0) s_row[tid / 8 + i * (C::NT / 8)] = unscale_of(e);
-        }
-        floatx4 cm = zero4();
-        for (int kt = 0;;) {
-            floatx4 m = zero4();
-#pragma unroll
-            for (int i = 0; i < C::W_PER; ++i)
-#pragma unroll
-                for (int u = 0; u < 4; ++u) m[u] = fmaxf(m[u], fabsf(wr[i][u]));
-            if (BN / 4 < 64) {
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-#pragma unroll
-                    for (int x = BN / 4; x < 64; x <<= 1) m[u] = fmaxf(m[u], __shfl_xor(m[u], x));
-            }
-            *reinterpret_cast<floatx4*>(s_max + wave * BN + nc) = m;
-            __syncthreads();
-            bool zero = false;
-#pragma unroll
-            for (int w = 0; w < C::NW; ++w) {
-                const floatx4 t = *reinterpret_cast<const floatx4*>(s_max + w * BN + nc);
-#pragma unroll
-                for (int u = 0; u < 4; ++u) m[u] = fmaxf(m[u], t[u]);
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                if (cm[u] == 0.f) cm[u] = m[u];
-                zero |= cm[u] == 0.f && nc < cols;
-            }
-            // the same answer in every wave: each sees all columns
-            if (!__any(zero) || ++kt >= nkt) {
-                if (kt > 0) load_w(0);
-                break;
-            }
-            __syncthreads();
-            load_w(kt);
-        }
-        floatx4 us;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const unsigned e = scale_exp(cm[u]);
-            sw[u] = scale_of(e);
-            us[u] = unscale_of(e);
-        }
-        if (tid < BN / 4) *reinterpret_cast<floatx4*>(s_col + nc) = us;
-    }
-
-    auto store = [&](u16* st) {
+    auto store = [&] {
         // k chunk q of a row holds k = 4q..4q+3; lane half h of step s takes
         // chunks 4s + h and 4s + h + 2 (the order W's transposed reads give)
         const int q = tid & 7;
         const int pos = (q >> 2) * 16 + (q & 1) * 8 + ((q >> 1) & 1) * 4;
 #pragma unroll
-        for (int i = 0; i < C::A_PER; ++i) {
-            uint2 t[2];
-            half_pair(ar[i][0] * sa[i], ar[i][1] * sa[i], t[0].x, t[1].x);
-            half_pair(ar[i][2] * sa[i], ar[i][3] * sa[i], t[0].y, t[1].y);
-            u16* p = st + (tid / 8 + i * (C::NT / 8)) * C::AP + pos;
-            *reinterpret_cast<uint2*>(p) = t[0];
-            *reinterpret_cast<uint2*>(p + C::APL) = t[1];
-        }
+        for (int i = 0; i < C::A_PER; ++i) store_terms(lds + (tid / 8 + i * (C::NT / 8)) * C::AP + pos, C::APL, ar[i]);
 #pragma unroll
-        for (int i = 0; i < C::W_PER; ++i) {
-            uint2 t[2];
-            half_pair(wr[i][0] * sw[0], wr[i][1] * sw[1], t[0].x, t[1].x);
-            half_pair(wr[i][2] * sw[2], wr[i][3] * sw[3], t[0].y, t[1].y);
-            u16* p = st + 2 * C::APL + (tid / (BN / 4) + i * (C::NT / (BN / 4))) * C::WP + nc;
-            *reinterpret_cast<uint2*>(p) = t[0];
-            *reinterpret_cast<uint2*>(p + C::WPL) = t[1];
-        }
+        for (int i = 0; i < C::W_PER; ++i)
+            store_terms(lds + 3 * C::APL + (tid / (BN / 4) + i * (C::NT / (BN / 4))) * C::WP + nc, C::WPL, wr[i]);
     };
 
     floatx16 acc[C::NB][C::MB];
@@ -510,69 +415,50 @@ __device__ __forceinline__ bool gemm_half_tile(const GemmArgs& g, unsigned char*
         for (int j = 0; j < C::MB; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-    auto compute = [&](const u16* st) {
+    auto compute = [&] {
         const int r = c & 15;
-        const u16* As = st + (wm0 + c) * C::AP + h * 8;
-        const u16* Ws = st + 2 * C::APL + (4 * h + (r >> 2)) * C::WP + wn0 + (c & 16) + 4 * (r & 3);
+        const u16* As = lds + (wm0 + c) * C::AP + h * 8;
+        const u16* Ws = lds + 3 * C::APL + (4 * h + (r >> 2)) * C::WP + wn0 + (c & 16) + 4 * (r & 3);
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
-            Half8 a[C::MB], w[C::NB];
+            Term8 a[C::MB], w[C::NB];
 #pragma unroll
             for (int j = 0; j < C::MB; ++j)
 #pragma unroll
-                for (int t = 0; t < 2; ++t)
-                    a[j].t[t] = *reinterpret_cast<const halfx8*>(As + t * C::APL + j * 32 * C::AP + s * 16);
+                for (int t = 0; t < 3; ++t)
+                    a[j].t[t] = *reinterpret_cast<const bf16x8*>(As + t * C::APL + j * 32 * C::AP + s * 16);
 #pragma unroll
             for (int i = 0; i < C::NB; ++i)
 #pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    const u16* p = Ws + t * C::WPL + s * 16 * C::WP + i * 32;
-                    w[i].t[t] = read_rows_tr(p, 8 * C::WP);
-                }
+                for (int t = 0; t < 3; ++t) w[i].t[t] = read_rows_tr(Ws + t * C::WPL + s * 16 * C::WP + i * 32, 8 * C::WP);
 #pragma unroll
             for (int i = 0; i < C::NB; ++i)
 #pragma unroll
-                for (int j = 0; j < C::MB; ++j) acc[i][j] = mfma_half(w[i], a[j], acc[i][j]);
+                for (int j = 0; j < C::MB; ++j) acc[i][j] = mfma_terms(w[i], a[j], acc[i][j]);
         }
     };
 
-    store(lds);
-    __syncthreads();
-    auto step = [&](int kt, auto stage_tag) {
-        constexpr int SB = decltype(stage_tag)::value;
-        if (kt + 1 < nkt) {
-            load_a(kt + 1);
-            load_w(kt + 1);
-        }
-        compute(lds + SB * C::STAGE16);
-        if (kt + 1 < nkt) store(lds + (1 - SB) * C::STAGE16);
+    if (tid == 0) *flag = 0;  // ordered by the loop's barriers
+    load(0);
+    for (int kt = 0; kt < nkt; ++kt) {
+        store();
         __syncthreads();
-    };
-    for (int kt = 0; kt < nkt; kt += 2) {
-        step(kt, std::integral_constant<int, 0>{});
-        if (kt + 1 < nkt) step(kt + 1, std::integral_constant<int, 1>{});
+        if (kt + 1 < nkt) load(kt + 1);
+        compute();
+        __syncthreads();
     }
 
     unsigned top = 0;
 #pragma unroll
     for (int i = 0; i < C::NB; ++i)
 #pragma unroll
-        for (int j = 0; j < C::MB; ++j) {
-            const float ua = s_row[wm0 + 32 * j + c];
+        for (int j = 0; j < C::MB; ++j)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const floatx4 uw = *reinterpret_cast<const floatx4*>(s_col + wn0 + 32 * i + 8 * q + 4 * h);
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    top = max(top, __float_as_uint(acc[i][j][4 * q + u]) & 0x7fffffffu);
-                    acc[i][j][4 * q + u] = acc[i][j][4 * q + u] * ua * uw[u];
-                }
+            for (int r = 0; r < 16; ++r) {
+                top = top_bits(top, acc[i][j][r]);
+                acc[i][j][r] *= kTermUnscale2;
             }
-        }
-    int* const flag = reinterpret_cast<int*>(s_max);  // zero after the loop's barriers
-    if (tid == 0) *flag = 0;
-    __syncthreads();
-    if (top >= 0x7f800000u) *flag = 1;  // inf or NaN
+    if (top >= kInfBits) *flag = 1;
     __syncthreads();
     if (*flag) return false;
     store_tile<C, true, BF16OUT>(g, acc, reinterpret_cast<float*>(lds_raw), m0 + wm0, n0 + wn0, wave, lane);
@@ -580,10 +466,10 @@ __device__ __forceinline__ bool gemm_half_tile(const GemmArgs& g, unsigned char*
 }
 
 template <int BM, int BN, int WM, int WN, bool BF16OUT, bool KF>
-__global__ __launch_bounds__(BM / WM * (BN / WN) * 64) void gemm_half_kernel(GemmArgs g) {
-    constexpr int FB = 2 * Cfg<BM, BN, WM, WN, 32>::STAGE * 4, HB = HalfCfg<BM, BN, WM, WN>::BYTES;
-    __shared__ __attribute__((aligned(16))) unsigned char lds[FB > HB ? FB : HB];
-    if (gemm_half_tile<BM, BN, WM, WN, BF16OUT, KF>(g, lds)) return;
+__global__ __launch_bounds__(BM / WM * (BN / WN) * 64) void gemm_terms_kernel(GemmArgs g) {
+    constexpr int FB = 2 * Cfg<BM, BN, WM, WN, 32>::STAGE * 4, TB = TermCfg<BM, BN, WM, WN>::BYTES;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[FB > TB ? FB : TB];
+    if (gemm_terms_tile<BM, BN, WM, WN, BF16OUT, KF>(g, lds)) return;
     __syncthreads();
     gemm_f32_tile<BM, BN, WM, WN, 32, true, BF16OUT, KF>(g, reinterpret_cast<float*>(lds));
 }
@@ -596,21 +482,21 @@ __global__ __launch_bounds__(BM / WM * (BN / WN) * 64) void gemm_f32_kernel(Gemm
 }
 
 template <int BM, int BN, int WM, int WN>
-hipError_t launch_half(const GemmArgs& g, hipStream_t s) {
+hipError_t launch_terms(const GemmArgs& g, hipStream_t s) {
     const int64_t tiles = (int64_t)((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN);
     if (tiles <= 0 || tiles > 0x7fffffff) return hipErrorInvalidConfiguration;
     const dim3 grid((unsigned)tiles), block(BM / WM * (BN / WN) * 64);
     const bool kf = g.K % 32 == 0;
     if (g.out_bf16) {
         if (kf)
-            hipLaunchKernelGGL((gemm_half_kernel<BM, BN, WM, WN, true, true>), grid, block, 0, s, g);
+            hipLaunchKernelGGL((gemm_terms_kernel<BM, BN, WM, WN, true, true>), grid, block, 0, s, g);
         else
-            hipLaunchKernelGGL((gemm_half_kernel<BM, BN, WM, WN, true, false>), grid, block, 0, s, g);
+            hipLaunchKernelGGL((gemm_terms_kernel<BM, BN, WM, WN, true, false>), grid, block, 0, s, g);
     } else {
         if (kf)
-            hipLaunchKernelGGL((gemm_half_kernel<BM, BN, WM, WN, false, true>), grid, block, 0, s, g);
+            hipLaunchKernelGGL((gemm_terms_kernel<BM, BN, WM, WN, false, true>), grid, block, 0, s, g);
         else
-            hipLaunchKernelGGL((gemm_half_kernel<BM, BN, WM, WN, false, false>), grid, block, 0, s, g);
+            hipLaunchKernelGGL((gemm_terms_kernel<BM, BN, WM, WN, false, false>), grid, block, 0, s, g);
     }
     return hipGetLastError();
 }
@@ -625,22 +511,25 @@ hipError_t launch_unaligned(const GemmArgs& g, hipStream_t s) {
     return hipGetLastError();
 }
 
-// 128 x 128 outputs per workgroup (four waves of 64 x 64: the fewest LDS reads
-// per MFMA that fit two workgroups on a CU) where those fill the CUs, else
-// 64 x 128 (eight waves of 32 x 32).  us, 128 x 128 against 64 x 128, by 128 x
-// 128 tiles: M 1024 N 768 K 256 (48) 16.8, 9.1; M 1024 N 2304 K 768 (144) 31.3,
-// 26.4; M 2048 N 2304 K 768 (288) 41.5, 46.0; M 8192 N 768 K 256 (384) 23.6,
-// 23.9; M 8192 N 2304 K 768 (1152) 122, 134.  256 x 128, 128 x 64, 64 x 64 and
-// eight waves on 128 x 128 were level or slower.
+// Tile shapes by how many 128 x 128 tiles there are for the 256 CUs: 128 x 128
+// (eight waves of 32 x 64, two workgroups per CU) where each CU gets one, 64 x 128
+// (eight of 32 x 32) for half as many, 64 x 64 (four of 32 x 32) below.  us, in this order:
+//   M 1024 N 768 K 256 (48 tiles of 128 x 128) 17.8, 12.3, 10.7; M 8192 N 256 K
+//   256 (128) 17.4, 12.8, 13.3; M 1024 N 2304 K 768 (144) 41.6, 41.4, 40.4; M
+//   2048 N 2304 K 768 (288) 63.3, 66.8, 65.2; M 8192 N 768 K 256 (384) 27.9,
+//   27.8, 30.4; M 8192 N 2304 K 768 (1152) 174, 200, 216; M 8192 N 3072 K 1024
+//   (1536) 280, 328, 352.
+// Four waves of 64 x 64 on 128 x 128 187 at 1152 tiles, 256 x 128 201; two LDS
+// stages, which leave one workgroup per CU, 216-266.
 // Each XCD takes a contiguous range of tiles (by_xcd) while W is small enough
-// to stay in its L2 beside the A rows: 122 -> 120 us at W of 7 MB, 23.6 -> 22.5
-// at 0.8 MB, level at 12 MB, 337 -> 356 at 50 MB.
+// to stay in its L2 beside the A rows.
 hipError_t launch_vec(const GemmArgs& in, hipStream_t s) {
     GemmArgs g = in;
     g.by_xcd = (int64_t)g.K * g.N <= (int64_t)2 << 20;
     if (g.K <= 0) return launch_unaligned(g, s);  // bias alone
     const int64_t tiles = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
-    return tiles >= 256 ? launch_half<128, 128, 64, 64>(g, s) : launch_half<64, 128, 32, 32>(g, s);
+    if (tiles >= 256) return launch_terms<128, 128, 32, 64>(g, s);
+    return tiles >= 128 ? launch_terms<64, 128, 32, 32>(g, s) : launch_terms<64, 64, 32, 32>(g, s);
 }
 
 }  // namespace
