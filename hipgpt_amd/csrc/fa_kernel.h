@@ -261,9 +261,11 @@ struct FaKernel {
         }
     };
 
-    // True (HALF only): this wave's results need the exact traits.
+    // False (HALF only, for all waves alike): the results need the exact traits,
+    // O and lse are not stored.  flags: two ints of LDS, zero, ordered by run's
+    // barriers.
     __device__ __forceinline__ static bool run(const AttnArgs& a, unsigned char* lds_raw, int* simd_slots,
-                                               int* v_seen = nullptr) {
+                                               int* flags = nullptr) {
         E* const lds = reinterpret_cast<E*>(lds_raw);
         const int tid = threadIdx.x;
         const int lane = tid & 63;
@@ -806,14 +808,10 @@ struct FaKernel {
         }
 
         // ---------------- epilogue: O = O^T / l (wave ks == 0) ----------------
-        // Row log-sum-exp (natural log) when asked for (no-probs path only):
-        // scores are in log2 units of scale * q.k, l = sum 2^(s - m) (without
-        // the factor 2^PSH, whose logarithm would cost the sum its last bits).
-        if (!PROBS && a.lse && ks == 0 && hf == 0 && qi < Sq)
-            a.lse[(int64_t)bh * Sq + qi] = ((m_run + PSH) + log2f(l_run * (1.f / (LAZY_SUM / kLazySum)))) * kLn2;
-        bool redo = false;
         if constexpr (HALF) {
-            redo = qreg.big();
+            // The exact traits start from Q again, and O may lie over Q: decide
+            // for the workgroup before any wave stores.
+            bool redo = qreg.big();
             if (ks == 0 && qi < Sq) {
                 const float linv = O_UNSCALE * __builtin_amdgcn_rcpf(fmaxf(l_run, 1e-20f));
                 unsigned top = 0;
@@ -823,9 +821,18 @@ struct FaKernel {
                     for (int r = 0; r < 16; ++r) top = max(top, __float_as_uint(o[db][r] * linv) & 0x7fffffffu);
                 redo |= top >= 0x7f800000u;  // inf or NaN
             }
+            if (redo) flags[0] = 1;
+            if (st.vtop >= kHalfVMin) flags[1] = 1;
+            __syncthreads();
+            if (flags[0] || !flags[1]) return false;
         }
+        // Row log-sum-exp (natural log) when asked for (no-probs path only):
+        // scores are in log2 units of scale * q.k, l = sum 2^(s - m) (without
+        // the factor 2^PSH, whose logarithm would cost the sum its last bits).
+        if (!PROBS && a.lse && ks == 0 && hf == 0 && qi < Sq)
+            a.lse[(int64_t)bh * Sq + qi] = ((m_run + PSH) + log2f(l_run * (1.f / (LAZY_SUM / kLazySum)))) * kLn2;
         if constexpr (O_TRANS) {
-            if constexpr (!O_TRANS_PAST) __syncthreads();  // the merge's reads of the area are done
+            if constexpr (!O_TRANS_PAST && !HALF) __syncthreads();  // the merge's reads of the area are done
             if (ks == 0) {
                 float* const X = reinterpret_cast<float*>(lds_raw + (O_TRANS_PAST ? MERGE_BYTES : 0)) + qs * QW * 36;
                 const float linv = O_UNSCALE * __builtin_amdgcn_rcpf(fmaxf(l_run, 1e-20f));
@@ -871,10 +878,7 @@ struct FaKernel {
                 }
             }
         }
-        if constexpr (HALF) {
-            if (st.vtop >= kHalfVMin) *v_seen = 1;
-        }
-        return redo;
+        return true;
     }
 };
 
@@ -906,11 +910,11 @@ void fa_fwd_kernel(AttnArgs a) {
         using KX = FaKernel<typename TR::exact, NQS, NKS, CAUSAL, PROBS, VEC, SRT>;
         __shared__ __attribute__((aligned(16)))
         unsigned char lds[K::LDS_BYTES > KX::LDS_BYTES ? K::LDS_BYTES : KX::LDS_BYTES];
-        __shared__ int redo, v_seen;
-        if (threadIdx.x == 0) redo = v_seen = 0;  // run's barriers order this before the stores below
-        if (K::run(a, lds, simd_slots, &v_seen)) redo = 1;
+        __shared__ int flags[2];
+        if (threadIdx.x == 0) flags[0] = flags[1] = 0;
+        if (K::run(a, lds, simd_slots, flags)) return;
         __syncthreads();
-        if (redo || !v_seen) KX::run(a, lds, simd_slots);
+        KX::run(a, lds, simd_slots);
     } else {
         __shared__ __attribute__((aligned(16))) unsigned char lds[K::LDS_BYTES];
         K::run(a, lds, simd_slots);

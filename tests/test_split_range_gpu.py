@@ -113,3 +113,18 @@ def test_outlier(shape, probs, value):
         elif np.isfinite(value):
             rel = D * 2.0 ** -24 * float(sc.abs().max()) * 1.4427
             assert float((o[bad] - want[bad]).abs().max()) <= float(x[2].abs().max()) * (rel + 1e-6)
+
+
+@pytest.mark.parametrize("shape", [SHAPES[i] for i in (0, 1, 4, 5, 6, 7, 9, 11)], ids=lambda s: "B%dH%dS%dD%d" % s)
+@pytest.mark.parametrize("causal", [False, True])
+def test_output_over_q(shape, causal):
+    """O in Q's place, also where a workgroup takes the second pass: it starts
+    from Q again, so nothing may be stored before."""
+    B, H, S, D = shape
+    for scale in ((1, 1, 1), (300, 1e-2, 1), (1, 1, 1e-6), (1, 1, 1e33)):
+        x = (make(*shape, seed=5) * torch.tensor(scale, dtype=torch.float32).view(3, 1, 1, 1, 1)).cuda()
+        q, k, v = x.unbind(0)
+        want = A.attention(q, k, v, causal=causal)
+        got = A.attention(q, k, v, out=q, causal=causal)
+        assert got.data_ptr() == x.data_ptr()
+        assert torch.equal(got, want), scale
