@@ -36,9 +36,6 @@ __device__ __forceinline__ bf16x8 as_bf16x8(uint4 v) {
     return r;
 }
 
-typedef short v4i16 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
-
 template <int D_>
 struct B16Traits {
     static constexpr int DP = D_;
@@ -66,7 +63,7 @@ struct B16Traits {
             q.v[s] = as_bf16x8(valid ? *reinterpret_cast<const uint4*>(p + 8 * s) : uint4{0u, 0u, 0u, 0u});
     }
 
-    __device__ __forceinline__ static float score_scale(const QReg&, float qscale) { return qscale; }
+    __device__ __forceinline__ static float score_scale(float qscale) { return qscale; }
     __device__ __forceinline__ static chunk from_u32x4(u32x4 v) { return uint4{v[0], v[1], v[2], v[3]}; }
 
     template <bool VEC>
@@ -121,7 +118,6 @@ struct B16Traits {
     struct PReg {
         bf16x8 s[2];
     };
-    template <bool SCALED = false>
     __device__ __forceinline__ static PReg to_p(const floatx16& p) {
         PReg pb;
 #pragma unroll

@@ -3,8 +3,8 @@
 // Replaces flash_attention_kernel<32|64> and multihead_attention_kernel_fallback
 // (HipGPT src/hip_kernels.cpp:263-325, :329-402) for head dims up to 128
 // (D = 16, 48, 96, ... run zero-padded to the next of 32/64/128).  The kernel
-// body is fa_kernel.h; this file supplies the operand traits -- F32HalfTraits
-// below, and F32Traits, the fp32 MFMA ones it falls back to:
+// body is fa_kernel.h; this file supplies the operand traits -- F32TermTraits
+// below, and F32Traits, the fp32 MFMA ones it falls back to and small grids run:
 //   * S^T = K Q^T on v_mfma_f32_32x32x2_f32.  Q is held in registers,
 //     pre-scaled by scale*log2(e) (so scores are already in the log2
 //     domain).  Lane (c, h) takes the contraction indices d = h*DP/2 + s:
@@ -28,9 +28,10 @@ namespace {
 
 using fa::BK;
 
-template <int DP_, bool VPRE_ = (DP_ <= 32), int SRES_ = (DP_ == 32 ? 4 : 0)>
+template <int DP_, int NBUF_>
 struct F32Traits {
     static constexpr int DP = DP_;
+    static constexpr int NBUF = NBUF_;
     using elem = float;
     using gelem = float;
     using chunk = floatx4;
@@ -66,7 +67,7 @@ struct F32Traits {
     __device__ __forceinline__ static chunk from_u32x4(u32x4 v) { return __builtin_bit_cast(chunk, v); }
 
     // Q already carries scale*log2(e).
-    __device__ __forceinline__ static float score_scale(const QReg&, float) { return 1.0f; }
+    __device__ __forceinline__ static float score_scale(float) { return 1.0f; }
 
     template <bool VEC>
     __device__ __forceinline__ static chunk load_chunk(const float* base, int64_t rowoff, int cc, int D, bool ok) {
@@ -109,45 +110,19 @@ struct F32Traits {
 
     // V^T operands of a tile: lane (c, hf) of block db needs
     // V[acc_key(t, hf)][db*32 + c], t = 0..15 -- four ds_read_b128 per block.
-    // VPRE: read before the softmax (VReg holds them) -- the streaming kernel
-    // at DP = 32; otherwise each block is read just
-    // before use.  That brings the streaming kernel at DP = 64 to 128 VGPRs:
-    // with WAVES_PER_EU = 4 two 8-wave workgroups share a CU (c3: 132 -> 128
-    // us; prefetching V under the same cap spills).
-    static constexpr bool VPRE = VPRE_;
-    static constexpr int WAVES_PER_EU = (DP == 64 && !VPRE) ? 4 : 1;
-    // With probs, rows of up to SRES stages keep their score tiles in
-    // registers between the two sweeps (DP = 32: 4 stages, Sk <= 256 at two
-    // key splits).
-    static constexpr int PROBS_RES_STAGES = SRES_;
     struct VReg {
-        floatx4 v[VPRE ? DP / 32 : 1][4];
         const float* vt;
     };
-    __device__ __forceinline__ static void load_block(floatx4 (&dst)[4], const float* Vt, int db, int c, int hf) {
-        const float* p = Vt + (db * 32 + c) * VTP + 4 * hf;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) dst[g] = *reinterpret_cast<const floatx4*>(p + 8 * g);
-    }
-    __device__ __forceinline__ static void load_v(VReg& vr, const float* Vt, int c, int hf) {
-        vr.vt = Vt;
-        if (VPRE)
-#pragma unroll
-            for (int db = 0; db < DP / 32; ++db) load_block(vr.v[VPRE ? db : 0], Vt, db, c, hf);
-    }
+    __device__ __forceinline__ static void load_v(VReg& vr, const float* Vt, int, int) { vr.vt = Vt; }
     using PReg = floatx16;
-    template <bool SCALED = false>
     __device__ __forceinline__ static const floatx16& to_p(const floatx16& p) { return p; }
     __device__ __forceinline__ static void pv(const VReg& vr, const floatx16& p, floatx16* o, int c, int hf) {
 #pragma unroll
         for (int db = 0; db < DP / 32; ++db) {
+            const float* const v = vr.vt + (db * 32 + c) * VTP + 4 * hf;
             floatx4 blk[4];
-            if (VPRE) {
 #pragma unroll
-                for (int g = 0; g < 4; ++g) blk[g] = vr.v[VPRE ? db : 0][g];
-            } else {
-                load_block(blk, vr.vt, db, c, hf);
-            }
+            for (int g = 0; g < 4; ++g) blk[g] = *reinterpret_cast<const floatx4*>(v + 8 * g);
 #pragma unroll
             for (int g = 0; g < 4; ++g)
 #pragma unroll
@@ -157,101 +132,72 @@ struct F32Traits {
     }
 };
 
-// The products on operands split into two fp16 terms (split.h), the traits
-// every problem runs unless its data need F32Traits (`exact`).  Tiles are two
-// row-major planes; operand layouts as in fa_bf16.hip (v_mfma_f32_32x32x16).
-//   Q: each row is scaled by the power of two that brings its largest
-//     magnitude to [2^7, 2^8), taken out of the scores by score_scale.
-//   K: times 2^6.  Whatever K's own scale, its terms are off by at most
-//     max(2^-24 |k|, 2^-31), so a score (log2 units) by a few 2^-31 |q|: the
-//     rows where that is not far below the rounding of the exponential have
-//     an entry of 16 or more (big()) and take the exact traits.
-//   V: times 2^8; exact traits if every |v| is below 2^-9.
-//   P: below 2^15 (kHalfPShift, kHalfPScale).
-// What overflows fp16 (|k| >= 1023, |v| >= 255) or is not finite ends in O as
-// inf or NaN and takes the exact traits.
-// B8 H12 S1024 D64 causal 124 -> 57 us, B4 H16 S2048 D128 causal 577 -> 219,
-// B32 H8 S256 D32 causal 15.6 -> 11.2, with probs unmasked 30.0 -> 22.9; error
-// against 64 bits 2.8e-7 -> 2.5e-7, 4.5e-7 -> 3.1e-7, 1.8e-7 -> 1.7e-7,
-// 4.2e-7 -> 3.6e-7.
-template <int DP_, int SRES_ = 0>
-struct F32HalfTraits {
+// The products on operands split into three bf16 terms (terms.h), the traits
+// every problem runs; a workgroup with a result that is not finite runs again
+// with F32Traits (`exact`).  Tiles are three row-major planes; operand layouts
+// as in fa_bf16.hip (v_mfma_f32_32x32x16).  Q, K, V and P carry 2^24 each, taken
+// out of the scores by score_scale and out of O in the epilogue.
+// Against fp32 MFMA, us: B8 H12 S1024 D64 causal 124 -> 86, B4 H16 S2048 D128 causal
+// 579 -> 351, B32 H8 S256 D32 causal 15.8 -> 14.1, with probs unmasked 30.2 -> 27.9,
+// 333 queries x 1357 keys B3 H12 D64 93 -> 42.  Bound by the matrix cores (six
+// MFMAs per product: 0.9-1.2 PFLOP/s at the two longest) and the vector ALUs
+// beside them (the softmax and the split of P, K and V).
+template <int DP_, int NBUF_ = 1, int SRES_ = 0, int WPE_ = (DP_ <= 64 ? 3 : 2)>
+struct F32TermTraits {
     static constexpr int DP = DP_;
+    static constexpr int NBUF = NBUF_;
     using elem = unsigned short;
     using gelem = float;
-    using exact = F32Traits<DP>;
+    using exact = F32Traits<DP, NBUF_>;
     using chunk = floatx4;
     static constexpr int KSTR = DP + 8;
     static constexpr int VRP = DP + 16;
     static constexpr int KPL = BK * KSTR;  // one term's plane
     static constexpr int VPL = BK * VRP;
-    static constexpr int KTILE = 2 * KPL;
-    static constexpr int VTILE = 2 * VPL;
-    static constexpr int WAVES_PER_EU = DP == 64 ? 3 : 2;
+    static constexpr int KTILE = 3 * KPL;
+    static constexpr int VTILE = 3 * VPL;
+    static constexpr int WAVES_PER_EU = WPE_;
     static constexpr int PROBS_RES_STAGES = SRES_;
 
     struct QReg {
-        Half8 v[DP / 16];
-        float unscale;
-        unsigned top;  // bits of the row's largest |q|
-        __device__ __forceinline__ bool big() const { return top >= 0x41800000u; }  // 16
+        Term8 v[DP / 16];
     };
 
     template <bool VEC>
     __device__ __forceinline__ static void load_q(QReg& q, const float* qrow, int hf, bool valid, int D, float qscale) {
         const float* p = qrow + hf * (DP / 2);
-        float x[DP / 2];
-        float mx = 0.f;
-#pragma unroll
-        for (int u = 0; u < DP / 2; u += 4) {
-            floatx4 t = {0.f, 0.f, 0.f, 0.f};
-            if (VEC) {
-                if (valid) t = *reinterpret_cast<const floatx4*>(p + u);
-            } else {
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (valid && hf * (DP / 2) + u + i < D) t[i] = p[u + i];
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                x[u + i] = t[i] * qscale;
-                mx = fmaxf(mx, fabsf(x[u + i]));
-            }
-        }
-        mx = fa::halves_max(mx);
-        q.top = __float_as_uint(mx);
-        // the row's largest magnitude to [2^7, 2^8); rows below 2^-64 as if at 2^-64
-        const unsigned e = max(q.top >> 23, 63u);
-        const float scale = __uint_as_float((261u - e) << 23);
-        q.unscale = __uint_as_float((e - 7u) << 23) * (1.f / fa::kHalfKScale);
+        const float scale = qscale * kTermScale;
 #pragma unroll
         for (int j = 0; j < DP / 16; ++j) {
-            float y[8];
+            float x[8];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) y[u] = x[8 * j + u] * scale;
-            q.v[j] = half8<false>(y, 1.f);
+            for (int u = 0; u < 8; u += 4) {
+                floatx4 t = {0.f, 0.f, 0.f, 0.f};
+                if (VEC) {
+                    if (valid) t = *reinterpret_cast<const floatx4*>(p + 8 * j + u);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (valid && hf * (DP / 2) + 8 * j + u + i < D) t[i] = p[8 * j + u + i];
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) x[u + i] = t[i] * scale;
+            }
+            q.v[j] = term8(x);
         }
     }
 
     __device__ __forceinline__ static chunk from_u32x4(u32x4 v) { return __builtin_bit_cast(chunk, v); }
-    __device__ __forceinline__ static float score_scale(const QReg& q, float) { return q.unscale; }
+    __device__ __forceinline__ static float score_scale(float) { return kTermUnscale2; }
     template <bool VEC>
     __device__ __forceinline__ static chunk load_chunk(const float* base, int64_t rowoff, int cc, int D, bool ok) {
-        return F32Traits<DP>::template load_chunk<VEC>(base, rowoff, cc, D, ok);
-    }
-    template <int PLANE>
-    __device__ __forceinline__ static void store_chunk(unsigned short* dst, const chunk& v, float s) {
-        uint2 w[2];
-        half_pair(v[0] * s, v[1] * s, w[0].x, w[1].x);
-        half_pair(v[2] * s, v[3] * s, w[0].y, w[1].y);
-#pragma unroll
-        for (int t = 0; t < 2; ++t) *reinterpret_cast<uint2*>(dst + t * PLANE) = w[t];
+        return exact::template load_chunk<VEC>(base, rowoff, cc, D, ok);
     }
     __device__ __forceinline__ static void store_k_chunk(unsigned short* Kt, int r, int cc, const chunk& v) {
-        store_chunk<KPL>(Kt + r * KSTR + cc * 4, v, fa::kHalfKScale);
+        store_terms(Kt + r * KSTR + cc * 4, KPL, v);
     }
     __device__ __forceinline__ static void store_vt_chunk(unsigned short* Vt, int r, int cc, const chunk& v) {
-        store_chunk<VPL>(Vt + r * VRP + cc * 4, v, fa::kHalfVScale);
+        store_terms(Vt + r * VRP + cc * 4, VPL, v);
     }
 
     __device__ __forceinline__ static floatx16 qk(const unsigned short* Kt, const QReg& q, int c, int hf) {
@@ -259,15 +205,16 @@ struct F32HalfTraits {
         floatx16 s;
 #pragma unroll
         for (int r = 0; r < 16; ++r) s[r] = 0.f;
-        Half8 k[DP / 16];
 #pragma unroll
         for (int j = 0; j < DP / 16; ++j) {
+            Term8 k;
 #pragma unroll
-            for (int t = 0; t < 2; ++t) k[j].t[t] = *reinterpret_cast<const halfx8*>(kr + t * KPL + 8 * j);
-            s = mfma_half_small(k[j], q.v[j], s);
+            for (int t = 0; t < 3; ++t) k.t[t] = *reinterpret_cast<const bf16x8*>(kr + t * KPL + 8 * j);
+            s = mfma_terms_small(k, q.v[j], s);
         }
+        asm volatile("" ::: "memory");  // the first terms are read again: held, they spill
 #pragma unroll
-        for (int j = 0; j < DP / 16; ++j) s = mfma_f16(k[j].t[0], q.v[j].t[0], s);
+        for (int j = 0; j < DP / 16; ++j) s = mfma_bf16(*reinterpret_cast<const bf16x8*>(kr + 8 * j), q.v[j].t[0], s);
         return s;
     }
 
@@ -277,24 +224,26 @@ struct F32HalfTraits {
     __device__ __forceinline__ static void load_v(VReg& vr, const unsigned short* Vt, int, int) { vr.vt = Vt; }
     // V terms of step s, block db: V[16s + 4hf + 0..3][db*32 + c] and the four
     // rows eight further on, transposed by ds_read_b64_tr_b16.
-    __device__ __forceinline__ static Half8 v_terms(const unsigned short* Vt, int db, int s, int c, int hf) {
+    __device__ __forceinline__ static Term8 v_terms(const unsigned short* Vt, int db, int s, int c, int hf) {
         const int r = c & 15;
         const unsigned short* p = Vt + (16 * s + 4 * hf + (r >> 2)) * VRP + db * 32 + (c & 16) + 4 * (r & 3);
-        Half8 v;
+        Term8 v;
 #pragma unroll
-        for (int t = 0; t < 2; ++t) v.t[t] = read_rows_tr(p + t * VPL, 8 * VRP);
+        for (int t = 0; t < 3; ++t) v.t[t] = read_rows_tr(p + t * VPL, 8 * VRP);
         return v;
     }
-    using PReg = HalfP;
-    template <bool SCALED = false>
+    using PReg = TermP;
     __device__ __forceinline__ static PReg to_p(const floatx16& p) {
-        return half_p<SCALED>(p, fa::kHalfPScale);
+        floatx16 x;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) x[r] = p[r] * kTermScale;
+        return term_p(x);
     }
     __device__ __forceinline__ static void pv(const VReg& vr, const PReg& pb, floatx16* o, int c, int hf) {
 #pragma unroll
         for (int db = 0; db < DP / 32; ++db)
 #pragma unroll
-            for (int s = 0; s < 2; ++s) o[db] = mfma_half(v_terms(vr.vt, db, s, c, hf), pb.s[s], o[db]);
+            for (int s = 0; s < 2; ++s) o[db] = mfma_terms(v_terms(vr.vt, db, s, c, hf), pb.s[s], o[db]);
     }
 };
 
@@ -303,38 +252,54 @@ struct F32HalfTraits {
 // device's 256 CUs.  Few: the keys of a row are split over up to four waves
 // and the workgroups are small, so that more CUs have work and a row's serial
 // chain is shorter.  Many: no key split (no merge, no wave idle in the
-// diagonal stages), two or three workgroups per CU.  SRES: probs rows of up
-// to SRES stages keep their scores in registers between the two sweeps.
-// us, shapes at n128 (head dim, entry, keys):
-//   D=32 causal, 256 keys: 2x2 9.2, 4x1 10.6 at 256; 14.8, 11.7 at 512; 1024
-//     keys: 1x4 13.6, 2x4 15.1, 2x2 17.8 at 64; 18.0, 15.2, 17.9 at 128; 2x2
-//     18.3, 4x1 24.7 at 256; 46.2, 41.1 at 1024.
-//   D=32 probs, 256 keys: 1x4 7.6, 2x2 9.7 at 64; 2x2 22.9, 4x1 29.1 at 512;
-//     1024 keys: 2x4 26.5, 2x2 31.2 at 128.
-//   D=64 causal, 256 keys: 1x4 10.0, 2x4 11.2, 4x2 11.7 at 64; 4x1 17.0, 4x2
-//     22.4 at 512; 1024 keys: 2x4 23.6, 2x2 27.3, 4x2 28.8 at 128; 4x2 37.7,
-//     4x1 39.9 at 384; 4x1 58.4, 4x2 68.3 at 768.
-//   D=64 probs, 256 keys: 2x2 33.9, 4x2 39.9, 4x1 45.0 at 512; 1024 keys: 2x4
-//     40.6, 4x2 49.5 at 128; 4x2 78, 4x1 90 at 256; level from 384 on.
-//   D=128 causal, 1024 keys: 2x2 51, 4x1 64, 8x1 74 at 128; 4x1 78, 8x1 81 at
-//     512; 8x1 136, 4x1 143 at 1024.  Probs, 256 keys: 2x2 22.5, 4x1 34 at
-//     128; 4x1 36, 2x2 39 at 256.
-template <int DP, int NQS, int NKS, int SRES = 0, bool VEC = true>
+// diagonal stages), two or three workgroups per CU.  One stage buffer (NBUF)
+// unless a second costs no workgroup.  SRES: probs rows of up to SRES stages
+// keep their scores in registers between the two sweeps.
+// us, shapes (x NBUF) at n128; c: causal, f: unmasked, p: unmasked with probs:
+//   D=32, 256 keys: 128 c 1x4 9.0, 2x2x2 9.5, 2x4 9.6, f 10.6, 9.2, 9.4, p 12.3,
+//     14.5, 15.6; 256 c 2x2x2 10.3, 4x2 11.4, f 12.1, 11.6, p 16.8, 20.8; 1024 c
+//     4x1x2 22.8, 4x2 25.0, 2x2x2 30.8, p 57.7, 61.1, 56.1.  1024 keys: 64 c 1x4
+//     18.1, 2x4 19.4, 2x2x2 22.5; 128 p 2x4 37.8, 1x4 45.7; 256 c 2x2x2 24.3, 2x4
+//     25.2, 4x2 29.0, f 34.9, 37.5, 30.8, p 69.5, 59.6, 65.6; 1024 c 4x2 60.4,
+//     4x1x2 62.9, 2x2x2 71.8.
+//   D=64, 256 keys: 128 2x2 14.0, 2x4 14.1, 4x2 16.9; 256 c 2x2 14.7, 4x2 17.5, f
+//     19.9, 18.8, p 25.6, 28.9; 1024 c 4x1 42.0, 8x1 54.4, 2x2 51.7.  1024 keys:
+//     128 2x4 32.5, 2x2 38.0, 4x2 45.8; 256 c 2x2 41.4, 2x4 42.6, 4x2 46.9, f 60.2,
+//     65.1, 52.4, p 98.6, 107.9, 92.6; 512 c 4x2 60.5, 4x1 69.3, f 104, 98.8; 768 c
+//     4x1 85.6, 4x1x2 89.3, 4x2 92.6, p 246, 264, 275.
+//   D=128, 256 keys: 128 2x2 26.4, 4x1x2 33.5; 256 2x2 38.1, 4x1x2 34.1; 512 4x1
+//     43.2, 8x1x2 43.6.  1024 keys: 256 c 2x2 86.4, 4x1x2 109, f 147, 109, p 219,
+//     170; 512 c 4x1 128, 8x1x2 132, f 185, 171, p 293, 297; 768 c 176, 185; 1024 c
+//     224, 199; 2048 keys: 1024 c 393, 351.
+template <int DP, int NQS, int NKS, int NBUF, int SRES = 0, int WPE = (DP <= 64 ? 3 : 2), bool VEC = true>
 hipError_t launch_shape(const AttnArgs& a, bool causal, bool probs, hipStream_t s) {
-    return fa::launch_fa_flags<F32HalfTraits<DP, SRES>, NQS, NKS, VEC>(a, causal, probs, s);
+    return fa::launch_fa_flags<F32TermTraits<DP, NBUF, SRES, WPE>, NQS, NKS, VEC>(a, causal, probs, s);
+}
+
+// Small grids over rows of 129 to 256 keys on fp32 MFMA itself, two stages of a 1 x
+// 4 workgroup: each call is one short chain of load, scores, softmax and product
+// per wave, which the terms' conversion lengthens.  us, terms against this, 16
+// and 64 blocks of 128 rows: D=32 with probs 8.5, 7.6 and 8.9, 8.0, causal 7.9,
+// 7.7 and 7.9, 7.4; D=64 level (12.7, 12.8; 12.5, 12.3).
+template <int DP>
+hipError_t launch_small(const AttnArgs& a, bool causal, bool probs, hipStream_t s) {
+    using T = F32Traits<DP, 2>;
+    if (probs)
+        return causal ? fa::launch_fa<T, 1, 4, true, true, true, 2>(a, s) : fa::launch_fa<T, 1, 4, false, true, true, 2>(a, s);
+    return causal ? fa::launch_fa<T, 1, 4, true, false, true>(a, s) : fa::launch_fa<T, 1, 4, false, false, true>(a, s);
 }
 
 // Head dims below the padded one and unaligned rows (guarded loads): two
 // shapes each, for grids that do and do not fill the device.
 hipError_t launch_guarded(const AttnArgs& a, bool causal, bool probs, int64_t n128, hipStream_t s) {
     switch (fa_f32_padded_dim(a.D)) {
-        case 32: return launch_shape<32, 2, 2, 4, false>(a, causal, probs, s);
+        case 32: return launch_shape<32, 2, 2, 2, 4, 1, false>(a, causal, probs, s);
         case 64:
-            return n128 <= 128 ? launch_shape<64, 2, 4, 0, false>(a, causal, probs, s)
-                               : launch_shape<64, 4, 2, 0, false>(a, causal, probs, s);
+            return n128 <= 128 ? launch_shape<64, 2, 4, 1, 0, 1, false>(a, causal, probs, s)
+                               : launch_shape<64, 4, 2, 1, 0, 1, false>(a, causal, probs, s);
         case 128:
-            return n128 <= 128 ? launch_shape<128, 2, 2, 0, false>(a, causal, probs, s)
-                               : launch_shape<128, 8, 1, 0, false>(a, causal, probs, s);
+            return n128 <= 128 ? launch_shape<128, 2, 2, 1, 0, 1, false>(a, causal, probs, s)
+                               : launch_shape<128, 8, 1, 1, 0, 1, false>(a, causal, probs, s);
         default: return hipErrorInvalidValue;
     }
 }
@@ -353,23 +318,30 @@ hipError_t launch_fa_f32(const AttnArgs& a, bool causal, bool vec, hipStream_t s
     const int64_t n128 = (int64_t)a.B * a.H * ((a.Sq + 127) / 128);
     const int Sk = a.Sk;
     if (!vec) return launch_guarded(a, causal, probs, n128, s);
+    const bool small = n128 <= 64 && Sk > 128 && Sk <= 256;
     switch (fa_f32_padded_dim(a.D)) {
         case 32:
-            if (n128 <= 64 && Sk > 128) return launch_shape<32, 1, 4, 2>(a, causal, probs, s);
-            if (n128 <= 128 && Sk > 256) return launch_shape<32, 2, 4, 2>(a, causal, probs, s);
-            if (n128 < 512 || probs) return launch_shape<32, 2, 2, 4>(a, causal, probs, s);
-            return launch_shape<32, 4, 1>(a, causal, probs, s);
+            if (small) return launch_small<32>(a, causal, probs, s);
+            if (n128 <= 64 || (n128 <= 128 && Sk <= 256 && (causal || probs)))
+                return launch_shape<32, 1, 4, 1, 2>(a, causal, probs, s);
+            if (n128 <= 128 && Sk > 256) return launch_shape<32, 2, 4, 1, 2>(a, causal, probs, s);
+            if (n128 <= 128 || (probs ? Sk <= 256 : causal && n128 <= 256))
+                return launch_shape<32, 2, 2, 2, 4>(a, causal, probs, s);
+            if (n128 >= 512 && Sk <= 256) return launch_shape<32, 4, 1, 2>(a, causal, probs, s);
+            return launch_shape<32, 4, 2, 1, 2>(a, causal, probs, s);
         case 64:
-            if (n128 <= 64 && Sk <= 256 && Sk > 128) return launch_shape<64, 1, 4, 2>(a, causal, probs, s);
-            if (n128 <= 128) return launch_shape<64, 2, 4>(a, causal, probs, s);
-            if (probs && Sk <= 256) return launch_shape<64, 2, 2, 4>(a, causal, probs, s);
+            if (small) return launch_small<64>(a, causal, probs, s);
+            if (n128 <= 128 && Sk > 256) return launch_shape<64, 2, 4, 1>(a, causal, probs, s);
+            if (n128 <= 128 || (n128 <= 256 && (causal || (probs && Sk <= 256))))
+                return launch_shape<64, 2, 2, 1, 4>(a, causal, probs, s);
             if (n128 <= 256 || (causal && n128 <= 512 && Sk > 512))
-                return launch_shape<64, 4, 2>(a, causal, probs, s);
-            return launch_shape<64, 4, 1>(a, causal, probs, s);
+                return launch_shape<64, 4, 2, 1>(a, causal, probs, s);
+            return launch_shape<64, 4, 1, 1>(a, causal, probs, s);
         case 128:
-            if (n128 <= 128) return launch_shape<128, 2, 2>(a, causal, probs, s);
-            if (n128 <= 512 || probs) return launch_shape<128, 4, 1>(a, causal, probs, s);
-            return launch_shape<128, 8, 1>(a, causal, probs, s);
+            if (n128 <= 128 || (n128 <= 256 && causal && Sk > 512)) return launch_shape<128, 2, 2, 1>(a, causal, probs, s);
+            if (n128 <= 256) return launch_shape<128, 4, 1, 2>(a, causal, probs, s);
+            if (n128 < 1024) return launch_shape<128, 4, 1, 1>(a, causal, probs, s);
+            return launch_shape<128, 8, 1, 2>(a, causal, probs, s);
         default: return hipErrorInvalidValue;
     }
 }

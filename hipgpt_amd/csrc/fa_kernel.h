@@ -26,7 +26,7 @@
 
 #include "common.h"
 #include "fa_common.h"
-#include "split.h"
+#include "terms.h"
 
 namespace hipgpt {
 namespace fa {
@@ -61,21 +61,20 @@ constexpr int kTransOwnMinDP = 128;
 // Start stagger only for grids of at most this many query blocks per (b, h).
 constexpr int kStaggerMaxBlocks = 4;
 
-// Traits of split operands (split.h; HALF) name the fp32 MFMA traits they
-// stand in for as `exact`; a workgroup whose data are outside the range the
-// split is good for runs again with those.
+// Traits of operands split into terms (terms.h; TERMS) name the fp32 MFMA traits
+// they stand in for as `exact`; a workgroup with a result that is not finite
+// runs again with those.
 template <class TR, class = void>
 struct exact_traits { using type = void; };
 template <class TR>
 struct exact_traits<TR, std::void_t<typename TR::exact>> { using type = typename TR::exact; };
 
-// Powers of two the operands carry so that both fp16 terms keep their bits
-// (split.h); Q rows carry one of their own (F32HalfTraits::load_q).
-constexpr float kHalfPShift = 7.f;     // exponentials up to 2^(kLazyMax + 7) = 2^15 < 65504
-constexpr float kHalfPScale = 16384.f; // normalised probs (<= 1) before the split
-constexpr float kHalfKScale = 64.f;    // K: |k| < 1023
-constexpr float kHalfVScale = 256.f;   // V: |v| < 255
-constexpr float kHalfVMin = 1.f / 512; // and at least one |v| this large
+// Stage buffers in LDS (traits may set NBUF): two, one barrier per stage; or one,
+// two barriers per stage and twice the workgroups per CU.
+template <class TR, class = void>
+struct stage_buffers { static constexpr int value = 2; };
+template <class TR>
+struct stage_buffers<TR, std::void_t<decltype(TR::NBUF)>> { static constexpr int value = TR::NBUF; };
 
 // SRT > 0 (probs only): when a wave's key tiles span at most SRT stages, the
 // max/sum sweep keeps every score tile in registers and the probs sweep reads
@@ -101,14 +100,15 @@ struct FaKernel {
     using E = typename TR::elem;    // staged operands (LDS)
     using GE = typename TR::gelem;  // K / V / Q in global memory
     static constexpr bool F32IN = sizeof(GE) == 4;
-    static constexpr bool HALF = !std::is_void_v<typename exact_traits<TR>::type>;
+    static constexpr bool TERMS = !std::is_void_v<typename exact_traits<TR>::type>;
 
-    // LDS: two stage buffers of NKS (K tile + V^T tile); the end-of-kernel
+    // LDS: NBUF stage buffers of NKS (K tile + V^T tile); the end-of-kernel
     // merge reuses the same memory.
+    static constexpr int NBUF = stage_buffers<TR>::value;
     static constexpr int STAGE_ELEMS = NKS * (TR::KTILE + TR::VTILE);
     static constexpr int STAGE_BYTES = STAGE_ELEMS * (int)sizeof(E);
     static constexpr int MERGE_BYTES = NKS > 1 ? NW * 64 * (16 * NDB + 2) * 4 : 0;  // key-split merge only
-    static constexpr int BASE_BYTES = (2 * STAGE_BYTES > MERGE_BYTES) ? 2 * STAGE_BYTES : MERGE_BYTES;
+    static constexpr int BASE_BYTES = (NBUF * STAGE_BYTES > MERGE_BYTES) ? NBUF * STAGE_BYTES : MERGE_BYTES;
     // Probs stores through a per-wave LDS transpose (see store_t): the score-
     // resident sweep borrows the idle K half of the stage buffers; the causal
     // probs sweeps at padded D >= kTransOwnMinDP (one workgroup
@@ -117,7 +117,7 @@ struct FaKernel {
     // 880 -> 867 us).  Unmasked there, the transpose measured slower (the
     // drop-in 1391 -> 1465 us).
     static constexpr bool TRANS_RES =
-        SRT > 0 && F32IN && TR::KTILE * (int)sizeof(E) >= QW * 36 * 4 && NW <= 2 * NKS;
+        SRT > 0 && F32IN && TR::KTILE * (int)sizeof(E) >= QW * 36 * 4 && NW <= NBUF * NKS;
     static constexpr bool TRANS_OWN = PROBS && CAUSAL && SRT <= 0 && F32IN && DP >= kTransOwnMinDP;
     static constexpr int LDS_BYTES = BASE_BYTES + (TRANS_OWN ? NW * QW * 36 * 4 : 0);
     // Without probs, the first stage stages K alone: the first Q K^T waits for
@@ -135,13 +135,9 @@ struct FaKernel {
     // the c1 and c3 shapes level; results unchanged bit for bit.  The
     // guarded-load instances (padded head dims) spill registers with it
     // (25 at D = 128) and keep the max test.
-    static constexpr bool SUM_CHECK = VEC && !(HALF && DP >= 128);
-    // Exponentials carry a factor 2^PSH without probs (it rides in m_run);
-    // with probs to_p<true> applies kHalfPScale.  Both, and V's, leave O in
-    // the epilogue.
-    static constexpr float PSH = HALF && !PROBS ? kHalfPShift : 0.f;
-    static constexpr float LAZY_SUM = HALF && !PROBS ? kLazySum * (float)(1 << (int)kHalfPShift) : kLazySum;
-    static constexpr float O_UNSCALE = !HALF ? 1.f : 1.f / kHalfVScale / (PROBS ? kHalfPScale : 1.f);
+    static constexpr bool SUM_CHECK = VEC && !(TERMS && DP >= 64);
+    // What O carries of the terms' scale (P and V).
+    static constexpr float O_UNSCALE = TERMS ? kTermUnscale2 : 1.f;
     // Causal grids larger than the device holds at once start their last
     // launch ranks (the shortest query blocks) as slots free, well into the
     // call, on Q rows nobody has read: each workgroup of rank r reads the Q
@@ -158,7 +154,7 @@ struct FaKernel {
     // stages are requested at once into the two stage buffers, so neither
     // sweep waits on a load after the first (each stage's loads were
     // otherwise requested one stage, ~0.5 us of compute, before use).
-    static constexpr bool LOAD_ALL = SRT == 2 && DP == 32;
+    static constexpr bool LOAD_ALL = SRT == 2 && DP == 32 && NBUF == 2;
     // O stores through LDS, one 32-dim block at a time (whole 128-byte row
     // segments per lane group), with a 32 x 36 scratch per storing wave
     // (ks == 0) inside the LDS already allocated: past the merge area when it
@@ -181,7 +177,6 @@ struct FaKernel {
     // guarded loads.)
     struct Stager {
         typename TR::chunk kr[PER], vr[PER];  // one stage of K and V chunks
-        mutable float vtop = 0.f;            // HALF: largest |v| stored
         int koff[PER], voff[PER];  // byte offsets of this thread's chunks from the stage's first row
         __amdgpu_buffer_rsrc_t krs, vrs;
         int kstage, vstage;        // bytes per stage of NKS*BK rows
@@ -251,23 +246,20 @@ struct FaKernel {
                 E* Kt = stage + kt * TR::KTILE;
                 E* Vt = stage + NKS * TR::KTILE + kt * TR::VTILE;
                 if (WK) TR::store_k_chunk(Kt, r, cc, kr[i]);
-                if (WV) {
-                    TR::store_vt_chunk(Vt, r, cc, vr[i]);
-                    if constexpr (HALF)
-                        vtop = fmaxf(fmaxf(vtop, fmaxf(fabsf(vr[i][0]), fabsf(vr[i][1]))),
-                                      fmaxf(fabsf(vr[i][2]), fabsf(vr[i][3])));
-                }
+                if (WV) TR::store_vt_chunk(Vt, r, cc, vr[i]);
             }
         }
     };
 
-    // False (HALF only, for all waves alike): the results need the exact traits,
-    // O and lse are not stored.  flags: two ints of LDS, zero, ordered by run's
+    // False (TERMS only, for all waves alike): the results need the exact traits,
+    // O and lse are not stored.  flag: an int of LDS, zero, ordered by run's
     // barriers.
     __device__ __forceinline__ static bool run(const AttnArgs& a, unsigned char* lds_raw, int* simd_slots,
-                                               int* flags = nullptr) {
+                                               int* flag = nullptr) {
         E* const lds = reinterpret_cast<E*>(lds_raw);
-        const int tid = threadIdx.x;
+        int tid = threadIdx.x;
+        // the second pass: nothing computed for the first stays live until it
+        if constexpr (F32IN && !TERMS) asm volatile("" : "+v"(tid));
         const int lane = tid & 63;
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
         const int c = lane & 31;
@@ -357,7 +349,7 @@ struct FaKernel {
 
         typename TR::QReg qreg;
         TR::template load_q<VEC>(qreg, Qp + (int64_t)qi * a.q_ts, hf, qi < Sq, a.D, a.qscale);
-        const float sc = TR::score_scale(qreg, a.qscale);
+        const float sc = TR::score_scale(a.qscale);
 
         floatx16 o[NDB];
 #pragma unroll
@@ -372,7 +364,7 @@ struct FaKernel {
         // instructions per score
         auto mask_edge = [&](floatx16& s, int t) {
             if (tr.edge(t, Sk, CAUSAL, qw0, off)) {
-                if constexpr (HALF) asm volatile("");
+                if constexpr (TERMS) asm volatile("");
                 mask_tile<CAUSAL>(s, t * BK, hf, qi, Sk, off);
             }
         };
@@ -444,12 +436,10 @@ struct FaKernel {
 
         // Exponentials of a score tile with the lazy rescale: the running max is
         // raised only when a row's tile max exceeds it by more than kLazyMax.
-        // m_run is the max less PSH, so that exponentials are at most
-        // 2^(kLazyMax + PSH).
         auto lazy_exp = [&](floatx16& sv) -> float {
             const float tmax = tile_max(sv) * sc;
-            if (__any(tmax > m_run + (kLazyMax + PSH))) {
-                const float m_new = vmax(m_run, tmax - PSH);
+            if (__any(tmax > m_run + kLazyMax)) {
+                const float m_new = vmax(m_run, tmax);
                 const float alpha = fast_exp2(m_run - m_new);
                 l_run *= alpha;
 #pragma unroll
@@ -468,13 +458,18 @@ struct FaKernel {
         };
 
         // ------------------------------------------------------------------
-        // One stage of compute on LDS buffer (i & 1).  MODE 0: online softmax
+        // One stage of compute on its LDS buffer.  MODE 0: online softmax
         // + PV.  MODE 1: max/sum only (SPILL: and the scores stored).  MODE 2:
         // probs store + PV with the final (m, l) (SPILL: from the stored scores).
+        auto buf_of = [](int i) { return NBUF == 2 ? (i & 1) * STAGE_ELEMS : 0; };
+        // before a stage is stored: with one buffer, the last one's reads are done
+        auto buf_free = [] {
+            if constexpr (NBUF == 1) __syncthreads();
+        };
         floatx16 s_next;  // SPILL, probs sweep: the next tile's stored scores, loaded one tile ahead
         auto compute = [&](auto mode_tag, int i, float mlog, float* prow, bool pvec) {
             constexpr int MODE = decltype(mode_tag)::value;
-            const E* cur = lds + (i & 1) * STAGE_ELEMS;
+            const E* cur = lds + buf_of(i);
             const int t = i * NKS + ks;
             if (t >= wtiles) return;
             floatx16 s;
@@ -499,7 +494,7 @@ struct FaKernel {
                         s[r] = fast_exp2(fmaf(s[r], sc, -m_run));
                         ls += s[r];
                     }
-                    if (__any(ls > LAZY_SUM)) {
+                    if (__any(ls > kLazySum)) {
                         asm volatile("" ::: "memory");  // re-read K: no copy of the first product stays live
                         s = tile_scores(cur, t);
                         ls = lazy_exp(s);
@@ -525,7 +520,7 @@ struct FaKernel {
                     store_t(Xown, prow - (int64_t)c * Sk, s, t * BK, pvec);
                 else if (qi < Sq)
                     store_probs_tile(prow, s, t * BK, hf, Sk, pvec);
-                TR::pv(vreg, TR::template to_p<true>(s), o, c, hf);
+                TR::pv(vreg, TR::to_p(s), o, c, hf);
             }
         };
 
@@ -573,14 +568,16 @@ struct FaKernel {
                     if (nstages > 1) st.template load<true, true>(1, tid);
                     __syncthreads();
                     first_pv(p0);
-                    if (nstages > 1) st.template store<true, true>(lds + STAGE_ELEMS, tid);
+                    buf_free();
+                    if (nstages > 1) st.template store<true, true>(lds + buf_of(1), tid);
                     __syncthreads();
                 }
                 for (int i = 1; i < nstages; ++i) {
                     if (i + 1 < nstages) st.template load<true, true>(i + 1, tid);
                     pf_issue(i);
                     compute(mode_tag, i, mlog, prow, pvec);
-                    if (i + 1 < nstages) st.template store<true, true>(lds + ((i + 1) & 1) * STAGE_ELEMS, tid);
+                    buf_free();
+                    if (i + 1 < nstages) st.template store<true, true>(lds + buf_of(i + 1), tid);
                     pf_keep(i);
                     __syncthreads();
                 }
@@ -596,7 +593,8 @@ struct FaKernel {
                 for (int i = 0; i + 1 < nstages; ++i) {
                     st.template load<WV, WK>(i + 1, tid);
                     compute(mode_tag, i, mlog, prow, pvec);
-                    st.template store<WV, WK>(lds + ((i + 1) & 1) * STAGE_ELEMS, tid);
+                    buf_free();
+                    st.template store<WV, WK>(lds + buf_of(i + 1), tid);
                     __syncthreads();
                 }
                 if (nstages > 0) {
@@ -609,7 +607,8 @@ struct FaKernel {
                     if (i + 1 < nstages) st.template load<WV, WK>(i + 1, tid);
                     if (MODE == 0) pf_issue(i);
                     compute(mode_tag, i, mlog, prow, pvec);
-                    if (i + 1 < nstages) st.template store<WV, WK>(lds + ((i + 1) & 1) * STAGE_ELEMS, tid);
+                    buf_free();
+                    if (i + 1 < nstages) st.template store<WV, WK>(lds + buf_of(i + 1), tid);
                     if (MODE == 0) pf_keep(i);
                     __syncthreads();
                 }
@@ -647,7 +646,7 @@ struct FaKernel {
                 } else {
                     if (qi < Sq) store_probs_tile(prow, p, t * BK, hf, Sk, pvec);
                 }
-                TR::pv(vreg, TR::template to_p<true>(p), o, c, hf);
+                TR::pv(vreg, TR::to_p(p), o, c, hf);
             }
         };
         auto sweep_res = [&](auto second_tag, float mlog, float* prow, bool pvec) {
@@ -685,9 +684,9 @@ struct FaKernel {
                     if (I < nstages) {
                         if (I + 1 < nstages) st.template load<SECOND, !SECOND>(I + 1, tid);
                         if (!SECOND && I == 0) st.template load<true, false>(0, tid);  // V of the probs sweep's first stage
-                        res_tile(second_tag, ic, lds + (I & 1) * STAGE_ELEMS, mlog, prow, pvec);
-                        if (I + 1 < nstages)
-                            st.template store<SECOND, !SECOND>(lds + ((I + 1) & 1) * STAGE_ELEMS, tid);
+                        res_tile(second_tag, ic, lds + buf_of(I), mlog, prow, pvec);
+                        buf_free();
+                        if (I + 1 < nstages) st.template store<SECOND, !SECOND>(lds + buf_of(I + 1), tid);
                         __syncthreads();
                     }
                 },
@@ -808,31 +807,26 @@ struct FaKernel {
         }
 
         // ---------------- epilogue: O = O^T / l (wave ks == 0) ----------------
-        if constexpr (HALF) {
+        if constexpr (TERMS) {
             // The exact traits start from Q again, and O may lie over Q: decide
             // for the workgroup before any wave stores.
-            bool redo = qreg.big();
             if (ks == 0 && qi < Sq) {
-                const float linv = O_UNSCALE * __builtin_amdgcn_rcpf(fmaxf(l_run, 1e-20f));
                 unsigned top = 0;
 #pragma unroll
                 for (int db = 0; db < NDB; ++db)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) top = max(top, __float_as_uint(o[db][r] * linv) & 0x7fffffffu);
-                redo |= top >= 0x7f800000u;  // inf or NaN
+                    for (int r = 0; r < 16; ++r) top = top_bits(top, o[db][r]);
+                if (top >= kInfBits) *flag = 1;
             }
-            if (redo) flags[0] = 1;
-            if (st.vtop >= kHalfVMin) flags[1] = 1;
             __syncthreads();
-            if (flags[0] || !flags[1]) return false;
+            if (*flag) return false;
         }
         // Row log-sum-exp (natural log) when asked for (no-probs path only):
-        // scores are in log2 units of scale * q.k, l = sum 2^(s - m) (without
-        // the factor 2^PSH, whose logarithm would cost the sum its last bits).
+        // scores are in log2 units of scale * q.k, l = sum 2^(s - m).
         if (!PROBS && a.lse && ks == 0 && hf == 0 && qi < Sq)
-            a.lse[(int64_t)bh * Sq + qi] = ((m_run + PSH) + log2f(l_run * (1.f / (LAZY_SUM / kLazySum)))) * kLn2;
+            a.lse[(int64_t)bh * Sq + qi] = (m_run + log2f(l_run)) * kLn2;
         if constexpr (O_TRANS) {
-            if constexpr (!O_TRANS_PAST && !HALF) __syncthreads();  // the merge's reads of the area are done
+            if constexpr (!O_TRANS_PAST && !TERMS) __syncthreads();  // the merge's reads of the area are done
             if (ks == 0) {
                 float* const X = reinterpret_cast<float*>(lds_raw + (O_TRANS_PAST ? MERGE_BYTES : 0)) + qs * QW * 36;
                 const float linv = O_UNSCALE * __builtin_amdgcn_rcpf(fmaxf(l_run, 1e-20f));
@@ -906,13 +900,13 @@ __attribute__((amdgpu_waves_per_eu(min_waves_per_eu<TR, NQS, NKS, CAUSAL, PROBS,
 void fa_fwd_kernel(AttnArgs a) {
     using K = FaKernel<TR, NQS, NKS, CAUSAL, PROBS, VEC, SRT>;
     __shared__ int simd_slots[NQS * NKS];
-    if constexpr (K::HALF) {
+    if constexpr (K::TERMS) {
         using KX = FaKernel<typename TR::exact, NQS, NKS, CAUSAL, PROBS, VEC, SRT>;
         __shared__ __attribute__((aligned(16)))
         unsigned char lds[K::LDS_BYTES > KX::LDS_BYTES ? K::LDS_BYTES : KX::LDS_BYTES];
-        __shared__ int flags[2];
-        if (threadIdx.x == 0) flags[0] = flags[1] = 0;
-        if (K::run(a, lds, simd_slots, flags)) return;
+        __shared__ int flag;
+        if (threadIdx.x == 0) flag = 0;
+        if (K::run(a, lds, simd_slots, &flag)) return;
         __syncthreads();
         KX::run(a, lds, simd_slots);
     } else {

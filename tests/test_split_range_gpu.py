@@ -1,15 +1,20 @@
-"""GPU tests of the split-operand forward (hipgpt_amd/csrc/split.h) at the
-edges of its range: fp32 operands run as two fp16 terms, with scales that hold
-for ordinary data, and a workgroup whose data lie outside runs again on fp32
-MFMA.  Here Q, K and V come at scales on both sides of every limit, with
-single outliers, and with infinities and NaN, in each workgroup shape of the
-dispatch and at ragged sizes.
+"""GPU tests of the fp32 forward on operands split into three bf16 terms
+(hipgpt_amd/csrc/terms.h): every operand bit is kept whatever the other values
+are, so Q, K and V come at scales far apart, with single outliers, single tiny
+or huge columns, rows and features, and with infinities, NaN and values past
+the terms' range (whose workgroups run again on fp32 MFMA), in each workgroup
+shape of the dispatch and at ragged sizes.
 
-Finite cases against float64.  A score is a D-term fp32 sum of magnitude at
-most smax (log2 units), so its error is below about D * 2^-24 * smax and that
-of P the same, relatively; O is a P-weighted mean of V, so its error is at most
-vmax times that plus the rounding of the products and of the sums over keys
-(tiles of 32 in sequence): bar = vmax * (2^-22 + D 2^-24 smax + Sk / 32 * 2^-24).
+Finite cases against float64, element by element and relative to what the
+element itself is made of.  A score (log2 units) is a D-term sum of magnitude
+abs = sum |q||k|: its products are each off by 2^-24 of their size, and six
+MFMAs per 16 dims add them in two groups, 12 D / 16 roundings of 2^-24 abs; the
+exponent's own rounding (|s| 2^-24) and that of v_exp_f32 (2^-22) come on top.
+An exponential is off by that times ln 2, relatively, and so is the row's sum,
+which adds up to Sk / 2 of them in one chain; P takes its logarithm into the
+exponent (a number below |s| + log2 Sk, rounded twice), O is off by the same
+share of sum_j P_j |v_j| of its column plus 12 Sk / 16 roundings of it (in the
+worst case; the bar is not reached).
 """
 import numpy as np
 import pytest
@@ -50,29 +55,65 @@ def ref(x, causal):
     return torch.matmul(p, v).permute(0, 2, 1, 3), p, s
 
 
-SCALES = [(1, 1, 1), (1e-6, 1, 1), (1, 1e-6, 1), (1, 1, 1e-6), (1, 1, 2.0 ** -9), (1, 1, 2.0 ** -12), (300, 1e-3, 1),
-          (1e-3, 900, 1), (1e-4, 1e4, 1), (1, 1, 200), (1, 1, 1e4), (1e-30, 1, 1e30), (1, 1, 0)]
+def bars(x, p, s):
+    """Bounds of |O - O64| and |P - P64| / P64, elementwise."""
+    q, k, v = (t.permute(0, 2, 1, 3).double() for t in x)
+    D, Sk = q.shape[-1], k.shape[-2]
+    mag = torch.matmul(q.abs(), k.abs().transpose(-1, -2)) * (1.4427 * D ** -0.5)
+    smax = torch.where(p > 0, s.abs() * 1.4427, 0.0).amax(-1, keepdim=True)
+    rel = (mag * (2 + 12 * D / 16) + s.abs().where(p > 0, 0.0) * 1.4427 + smax) * 2.0 ** -24 * 0.6932 + 2.0 ** -22
+    row = torch.where(p > 2.0 ** -60, rel, 0.0).amax(-1, keepdim=True) + Sk / 2 * 2.0 ** -24  # of the row's sum
+    o = torch.matmul(p * (rel + row + (2 + 12 * Sk / 16) * 2.0 ** -24), v.abs())
+    return o.permute(0, 2, 1, 3), rel + row + 2 * (smax + np.log2(Sk)) * 2.0 ** -24 * 0.6932
+
+
+SCALES = [(1, 1, 1), (1e-6, 1, 1), (1, 1e-6, 1), (1, 1, 1e-6), (1, 1, 2.0 ** -12), (300, 1e-3, 1), (1e-3, 900, 1),
+          (1e-4, 1e4, 1), (1, 1, 200), (1, 1, 1e15), (1e-30, 1, 1e30), (1e-30, 1e30, 1e-30), (1, 1, 0)]
+
+
+def check(x, causal, probs, tag):
+    o, p = run(x, causal, probs)
+    want, pw, s = ref(x, causal)
+    bo, bp = bars(x, pw, s)
+    floor = 2.0 ** -126 * x.shape[2]  # exponentials below fp32's smallest normal are 0
+    err = (o - want).abs() - floor * x[2].double().abs().amax(1, keepdim=True)
+    print(tag, tuple(x.shape[1:]), causal, probs, "%.3f of the bar" % float((err / bo.clamp_min(1e-300)).max()), flush=True)
+    assert (err <= bo + 1e-44).all()
+    if probs:
+        assert ((p - pw).abs() <= pw * bp + 2.0 ** -126).all()
 
 
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "B%dH%dS%dD%d" % s)
 @pytest.mark.parametrize("probs", [False, True])
 def test_scales(shape, probs):
     B, H, S, D = shape
-    for i, (sq, sk, sv) in enumerate(SCALES):
-        if B > 8 and i not in (0, 3, 6, 7):
+    for i, scale in enumerate(SCALES):
+        if B > 8 and i not in (0, 3, 5, 6):
             continue
-        x = make(*shape, seed=i) * torch.tensor([sq, sk, sv], dtype=torch.float32).view(3, 1, 1, 1, 1)
-        causal = i % 2 == 0
-        o, p = run(x, causal, probs)
-        want, pw, s = ref(x, causal)
-        smax = float(s[s > -1e300].abs().max()) * 1.4427
-        rel = 2.0 ** -22 + D * 2.0 ** -24 * smax + S / 32 * 2.0 ** -24
-        vmax = float(x[2].abs().max())
-        err = float((o - want).abs().max())
-        print(shape, probs, (sq, sk, sv), err, vmax * rel, flush=True)
-        assert err <= vmax * rel
-        if probs:
-            assert float((p - pw).abs().max()) <= rel
+        x = make(*shape, seed=i) * torch.tensor(scale, dtype=torch.float32).view(3, 1, 1, 1, 1)
+        check(x, i % 2 == 0, probs, scale)
+
+
+@pytest.mark.parametrize("shape", [SHAPES[i] for i in (0, 1, 3, 5, 6, 7, 9, 12)], ids=lambda s: "B%dH%dS%dD%d" % s)
+@pytest.mark.parametrize("probs", [False, True])
+def test_mixed_scales(shape, probs):
+    B, H, S, D = shape
+    for r in (2.0 ** 14, 2.0 ** 22, 2.0 ** 40):
+        x = make(*shape, seed=20)
+        x[0, ..., 0] *= r  # a feature large in Q and small in K
+        x[1, ..., 0] /= r
+        check(x, True, probs, "feature times %g" % r)
+    for r in (1e-5, 1e-10, 1e-30):
+        x = make(*shape, seed=21)
+        x[2, ..., 1] *= r  # a small column of V
+        x[2, :, :, :, 3] *= 1 / r ** 0.5
+        check(x, False, probs, "column of V times %g" % r)
+        x = make(*shape, seed=22)
+        x[2, :, :32] *= r  # causal: rows that see the small values only
+        check(x, True, probs, "first rows of V times %g" % r)
+    x = make(*shape, seed=23) * torch.tensor([1, 1, 1e-7], dtype=torch.float32).view(3, 1, 1, 1, 1)
+    x[2, 0, S - 1, 0, 0] = 2e-3
+    check(x, True, probs, "one larger value of V")
 
 
 @pytest.mark.parametrize("shape", [SHAPES[i] for i in (0, 1, 5, 6, 9, 12)], ids=lambda s: "B%dH%dS%dD%d" % s)
