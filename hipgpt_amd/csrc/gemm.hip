@@ -20,11 +20,11 @@
 //
 // gemm_terms_tile runs every problem with 16-byte rows on operands split into
 // three bf16 terms (terms.h; v_mfma_f32_32x32x16_bf16, six per product).  Against
-// the fp32 tile, us, and error against 64 bits: M 8192 N 2304 K 768 227 -> 174,
-// 3.5e-7 -> 3.0e-7; M 8192 N 768 K 256 30.0 -> 27.9, 2.0e-7 -> 1.7e-7; M 1024 N
-// 768 K 256 13.2 -> 10.7.  Bound by the matrix cores and, in turn with them, the
-// conversion of the next k-tile: six MFMAs per product at 174 us are 1.0
-// PFLOP/s, of the 1.62 that bf16 MFMAs alone reach on random data.
+// the fp32 tile, us, and error against 64 bits: M 8192 N 2304 K 768 227 -> 173,
+// 3.5e-7 -> 1.2e-7; M 8192 N 768 K 256 30.0 -> 28.2, 2.0e-7 -> 6.9e-8; M 1024 N
+// 768 K 256 13.2 -> 10.8.  Bound by the matrix cores and, in turn with them, the
+// conversion of the next k-tile: six MFMAs per product at 173 us are 1.0
+// PFLOP/s of the 1.62 that bf16 MFMAs alone reach on random data.
 //
 // gemm_f32_tile (v_mfma_f32_32x32x2_f32) takes tiles with a result that is not
 // finite on the terms, and operands without 16-byte rows:
@@ -408,13 +408,16 @@ __device__ __forceinline__ bool gemm_terms_tile(const GemmArgs& g, unsigned char
             store_terms(lds + 3 * C::APL + (tid / (BN / 4) + i * (C::NT / (BN / 4))) * C::WP + nc, C::WPL, wr[i]);
     };
 
-    floatx16 acc[C::NB][C::MB];
+    // the small terms have sums of their own: an addition rounds at the size the
+    // sum has, and these are 2^-8 of the others (M 8192 N 2304 K 768: 174 us and
+    // 3.0e-7 in one sum, 173 and 1.2e-7 so)
+    floatx16 acc[C::NB][C::MB], low[C::NB][C::MB];
 #pragma unroll
     for (int i = 0; i < C::NB; ++i)
 #pragma unroll
         for (int j = 0; j < C::MB; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = low[i][j][r] = 0.f;
     auto compute = [&] {
         const int r = c & 15;
         const u16* As = lds + (wm0 + c) * C::AP + h * 8;
@@ -434,7 +437,10 @@ __device__ __forceinline__ bool gemm_terms_tile(const GemmArgs& g, unsigned char
 #pragma unroll
             for (int i = 0; i < C::NB; ++i)
 #pragma unroll
-                for (int j = 0; j < C::MB; ++j) acc[i][j] = mfma_terms(w[i], a[j], acc[i][j]);
+                for (int j = 0; j < C::MB; ++j) {
+                    low[i][j] = mfma_terms_small(w[i], a[j], low[i][j]);
+                    acc[i][j] = mfma_bf16(w[i].t[0], a[j].t[0], acc[i][j]);
+                }
         }
     };
 
@@ -455,6 +461,7 @@ __device__ __forceinline__ bool gemm_terms_tile(const GemmArgs& g, unsigned char
         for (int j = 0; j < C::MB; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
+                acc[i][j][r] += low[i][j][r];
                 top = top_bits(top, acc[i][j][r]);
                 acc[i][j][r] *= kTermUnscale2;
             }
