@@ -7,7 +7,7 @@
 //   Dq_i = sum_j P_ij (dO_i . V_j)       (= dO_i . (P V)_i)
 //   dS   = P o (dO V^T - Dq)
 //   dQ = c dS K,   dK = c dS^T Q,   dV = P^T dO
-// Head dims up to 128 with 16-byte aligned rows run bwd_half.h (or, at S <=
+// Head dims up to 128 with 16-byte aligned rows run bwd_terms.h (or, at S <=
 // 256, one workgroup per (b, h): bwd_bh.h, bwd_bh64.h), 256 bwd_wide.h; the
 // kernels below serve every other problem.  Two kernels,
 // every gradient element written exactly once (no atomics, no memset):
@@ -24,7 +24,7 @@
 // diagonal, where a causal forward wrote zeros.
 #include "bwd_bh.h"
 #include "bwd_bh64.h"
-#include "bwd_half.h"
+#include "bwd_terms.h"
 #include "bwd_tiled.h"
 #include "bwd_wide.h"
 #include "common.h"
@@ -318,22 +318,21 @@ bool bwd_tiled_ok(const BwdArgs& a) {
 }
 
 // The one-workgroup-per-(b, h) kernels (S <= 256, fp32 MFMA, no workspace, each
-// stored P read once) against the query-/key-stationary pair on split operands
-// (P read twice).  The drop-in call keeps them for every shape they took
-// before, since its other kernels need a workspace that it may have to
-// allocate: D = 32, and D = 64 where the (b, h) pairs fill the CUs.  Else, us at
-// H = 8, per-(b, h) against pair:
-//   D = 64 causal stored probs, S = 64: B 2 14.2, 15.9; S = 128: B 2 25.5, 24.0,
-//     B 8 26.3, 26.4, B 32 28.8, 31.7; S = 256: B 2 62, 37, B 8 63, 41, B 32
-//     68, 66 (kept: the same bits as the drop-in there).
-//   D = 32 from lse, forward included, S = 256: B 32 44.0, 46.7, B 64 88.8, 98.4;
-//     S = 128: B 32 26.9, 23.1, B 64 48, 40; with fewer (b, h) than CUs S = 256
-//     B 8 36, 24.
-//   D = 64 from lse: the pair everywhere (S = 256 B 32 105, 90).
+// stored P read once) against the query-/key-stationary pair on bf16 terms (P
+// read twice).  The drop-in call keeps them for every shape they took before,
+// since its other kernels need a workspace that it may have to allocate.  us at
+// H = 8, per-(b, h) against pair, causal:
+//   D = 32 stored probs, S = 128: B 2 16.0, 22.5, B 64 34.8, 36.7; S = 256: B 2
+//     36.7, 39.1, B 32 39.6, 49.6.  From lse, S = 128: B 8 18.7, 13.0, B 32 20.1,
+//     20.2; S = 192: B 32 26.6, 33.9; S = 256: B 16 31.1, 25.1, B 32 32.8, 46.2.
+//   D = 64 stored probs, S = 128: B 2 25.5, 31.5, B 64 55.6, 57.1; S = 192: B 8
+//     44.2, 43.9; S = 256: B 2 62.7, 54.0, B 32 68.1, 75.1; unmasked, S = 128: B 2
+//     26.1, 32.4; S = 256: B 16 79.9, 67.8, B 32 86.1, 99.5.
+//   D = 64 from lse: the pair everywhere.
 static bool bh_better(const BwdArgs& a) {
     const bool full = (int64_t)a.B * a.H >= device_cus();
     if (!a.probs) return a.D == 32 && a.S > 128 && full;
-    return a.D == 32 || full || (a.causal && a.S <= 128);
+    return a.D == 32 || full || a.S <= 128;
 }
 
 // The head-dim-split kernels of bwd_wide.h: D % 4 == 0 up to 256, 16-byte
@@ -359,17 +358,19 @@ hipError_t launch_attn_bwd(const BwdArgs& a, hipStream_t s) {
     if (bwd_tiled_ok(a)) {
         if (bh_better(a) && bwd::bh_ok(a)) return bwd::launch_bh(a, s);
         if (bh_better(a) && bwd::bh_probs64_ok(a)) return bwd::launch_bh64(a, s);
-        return a.D == 32 ? bwd::launch_half<32, 4, 1, true>(a, s) : bwd::launch_half<64, 4, 1, true>(a, s);
+        return a.D == 32 ? bwd::launch_terms<32, 4, 1, true>(a, s) : bwd::launch_terms<64, 4, 1, true>(a, s);
     }
     if (bwd_wide_ok(a)) {
-        if (a.D <= 32) return bwd::launch_half<32, 4, 1, false>(a, s);
-        if (a.D <= 64) return bwd::launch_half<64, 4, 1, false>(a, s);
-        // 64-row blocks until 128-row ones give every CU one (one 8-wave
-        // workgroup per CU): 8 (b, h) of 1024 rows with stored probs 201 -> 178
-        // us, 32 232 -> 225; with more, 128-row blocks read each tile half as often
-        if (a.D <= 128)
-            return (int64_t)((a.S + 127) / 128) * a.B * a.H <= 256 ? bwd::launch_half<128, 2, 2, false>(a, s)
-                                                                   : bwd::launch_half<128, 4, 2, false>(a, s);
+        if (a.D <= 32) return bwd::launch_terms<32, 4, 1, false>(a, s);
+        if (a.D <= 64) return bwd::launch_terms<64, 4, 1, false>(a, s);
+        // 64-row blocks where 128-row ones (n128) leave CUs idle.  us, 64 against
+        // 128 rows: 128 stored causal 253, 314, lse causal 274, 345; 256 163, 177 and
+        // 187, 207, but unmasked 282, 195 and 300, 216; 512 222, 174.
+        if (a.D <= 128) {
+            const int64_t n128 = (int64_t)((a.S + 127) / 128) * a.B * a.H;
+            return n128 <= 128 || (a.causal && n128 <= 256) ? bwd::launch_terms<128, 2, 2, false>(a, s)
+                                                            : bwd::launch_terms<128, 4, 2, false>(a, s);
+        }
         return bwd::launch_wide<256, 2, 4, 1>(a, s);
     }
     if (a.D <= 32) return launch_dp<32>(a, s);

@@ -1,6 +1,6 @@
 // bwd_tiled.h -- LDS-tiled MFMA kernels of the attention backward on the
 // forward's probabilities (HipGPT src/hip_kernels.cpp:1159-1272), for head
-// dims 32 and 64 with 16-byte aligned rows.  The workgroups of bwd_half.h run
+// dims 32 and 64 with 16-byte aligned rows.  The workgroups of bwd_terms.h run
 // them where their split operands do not hold the data.
 //
 // Math per (b, h), scale c = 1/sqrt(D):
@@ -130,7 +130,9 @@ struct BwdQ {
 
     // Workgroup `rank` of the nqb query blocks of problem bh.
     __device__ __forceinline__ static void run(const BwdArgs& a, float* lds, int* simd_slots, int nqb, int bh, int rank) {
-        const int tid = threadIdx.x, lane = tid & 63;
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));  // as a second pass: nothing of the first stays live for it
+        const int lane = tid & 63;
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
         const int c = lane & 31, hf = lane >> 5;
         const int qb = CAUSAL ? nqb - 1 - rank : rank;
@@ -376,7 +378,9 @@ struct BwdKV {
 
     // Workgroup `rank` (the key block) of the nkb key blocks of problem bh.
     __device__ __forceinline__ static void run(const BwdArgs& a, float* lds, int* simd_slots, int nkb, int bh, int rank) {
-        const int tid = threadIdx.x, lane = tid & 63;
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));  // as a second pass: nothing of the first stays live for it
+        const int lane = tid & 63;
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
         const int c = lane & 31, hf = lane >> 5;
         const int kb = rank;  // key block; causal: block 0 sees the most query tiles and launches first

@@ -4,7 +4,7 @@
 // and 256 (whose per-wave accumulators and dO / V rows would not fit one
 // wave's registers) and head dims below 64 that are not 32 or 64, any D with
 // D % 4 == 0 and 16-byte aligned rows.  Head dims above 128 run them as
-// kernels; below, the workgroups of bwd_half.h where their split operands do
+// kernels; below, the workgroups of bwd_terms.h where their split operands do
 // not hold the data.
 //
 // Same math and the same two kernels as bwd_tiled.h (query-stationary dQ and
@@ -57,7 +57,9 @@ struct WideQ {
     static constexpr int LDS_FLOATS = NBUF * STAGE + XCH;
 
     __device__ __forceinline__ static void run(const BwdArgs& a, float* lds, int nqb, int bh, int rank) {
-        const int tid = threadIdx.x, lane = tid & 63;
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));  // as a second pass: nothing of the first stays live for it
+        const int lane = tid & 63;
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
         const int c = lane & 31, hf = lane >> 5;
         const int sb = wave / DH, dh = wave % DH;
@@ -235,7 +237,9 @@ struct WideKV {
     static_assert(STAGE % 4 == 0, "16-byte aligned stage buffers");
 
     __device__ __forceinline__ static void run(const BwdArgs& a, float* lds, int bh, int rank) {
-        const int tid = threadIdx.x, lane = tid & 63;
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));  // as a second pass: nothing of the first stays live for it
+        const int lane = tid & 63;
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
         const int c = lane & 31, hf = lane >> 5;
         const int sb = wave / DH, dh = wave % DH;
