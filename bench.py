@@ -1,13 +1,16 @@
 #!/usr/bin/env python3
 """Benchmark of the MI355X attention forward (HipGPT's hot path) on one GPU.
 
-Headline (BASELINE.json metric): causal attention forward TFLOP/s and the
-fraction of the fp32 MFMA roofline at B32 H8 S256 D32 (config c1), inputs
+Headline: causal attention forward TFLOP/s and the fraction of the roofline of
+fp32 products on the matrix cores at B32 H8 S256 D32 (config c1), inputs
 resident in HBM.  One step = one attention forward over the whole batch.
-The other BASELINE configs, the drop-in contract (non-causal + probs, the
-call HipGPT makes) at every config, and the neighbouring kernels are timed
-the same way and reported under "configs"; the oracle's scalar restatement is
-timed on the host cores as "cpu_baseline" for c1..c5.
+The other configs, the drop-in contract (non-causal + probs, the call HipGPT
+makes) at every config, and the neighbouring kernels are timed the same way; the
+oracle's scalar restatement is timed on the host cores for c1..c5.
+
+stdout is one JSON line of under 4 KB: the headline, and per config under
+"configs" its microseconds per call and roofline fraction.  stderr has a readable
+line per config; --details FILE takes everything measured, as JSON.
 
 Timing protocol, per config:
   * Input and output buffers are allocated in R independent sets, R chosen so
@@ -23,7 +26,7 @@ Timing protocol, per config:
   * "dist_us": p10 / p50 / p90 over max(steps, 100) calls, each between its
     own pair of events (rotating sets).
 
-Usage: python bench.py [--gpus 1] [--steps K] [--warmup W] [--only c1,c3] [--no-cpu] [--no-hot]
+Usage: python bench.py [--gpus 1] [--steps K] [--warmup W] [--only c1,c3] [--no-cpu] [--no-hot] [--details FILE]
 """
 import argparse
 import json
@@ -36,8 +39,11 @@ import time
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
-PEAK_F32_MFMA = 157.3e12   # MI355X dense fp32 matrix, FLOP/s
-PEAK_BF16_MFMA = 2.5e15    # dense bf16 matrix
+PEAK_BF16_MFMA = 2.5e15    # MI355X dense bf16 matrix, FLOP/s
+# fp32 products at fp32 accuracy: six bf16 MFMAs each (hipgpt_amd/csrc/terms.h),
+# 2.6 times the dense fp32 matrix rate
+PEAK_F32_MFMA = PEAK_BF16_MFMA / 6
+RATE_F32_MFMA = 157.3e12   # dense fp32 matrix
 PEAK_HBM = 8.0e12          # HBM3E bytes/s
 METRIC = "causal attention fwd TFLOP/s + % of MFMA roofline on 1 MI355X (B32 H8 S256 D32)"
 ROTATE_BYTES = 1 << 30     # buffer sets per config hold at least this much together
@@ -443,6 +449,51 @@ def read_traffic(name):
         return json.load(f).get("hbm_bytes_per_launch")
 
 
+def headline(steps, warmup, results, cpu):
+    """The JSON line: c1 and, in short, every config of `results`."""
+    head = results.get("c1", {})
+    line = {
+        "metric": METRIC,
+        "value": head.get("tflops"),
+        "unit": "TFLOP/s",
+        "n_gpus": 1,
+        "steps": steps,
+        "warmup": warmup,
+        "ms_per_step": round(head["us_per_call"] / 1e3, 6) if "us_per_call" in head else None,
+        "higher_is_better": True,
+        "scaling": "weak",
+        "vs_baseline": None,
+        "dtype": "fp32",
+        "data": "synthetic N(0,1) Q/K/V resident in HBM (planar [3][B*S][E] buffer, seeded; calls rotate "
+                "over buffer sets totalling >= 1 GiB so operands come from HBM, not the Infinity Cache)",
+        "config": {"model": "c1: causal self-attention forward, fp32, B=32 H=8 S=256 D=32 (E=256), "
+                            "no probs output", "global_batch": 32, "seq_len": 256, "B": 32, "H": 8, "S": 256, "D": 32,
+                   "parallelism": "single GPU"},
+    }
+    if "us_per_call" in head:
+        flops, _ = work(CONFIGS["c1"])
+        ach = flops / (head["us_per_call"] * 1e-6)
+        line["roofline"] = {
+            "bound": "mfma", "achieved": round(ach / 1e12, 3), "peak": PEAK_F32_MFMA / 1e12,
+            "unit": "TFLOP/s", "frac": round(ach / PEAK_F32_MFMA, 4),
+            "frac_of_fp32_mfma": round(ach / RATE_F32_MFMA, 4), "traffic": read_traffic("c1"),
+        }
+    if cpu is not None:
+        _, ncores, cfgs = cpu
+        c1 = cfgs["c1"]["one_thread"]
+        line["cpu_baseline"] = {
+            "value": round(c1["gflops"] / 1e3, 6), "unit": "TFLOP/s", "cores": 1, "kind": "port",
+            "sample": f"c1 through the oracle's scalar restatement of flash_attention_kernel<32>: {c1['pairs']} of "
+                      f"{c1['of_pairs']} (b,h) pairs, median of {c1['runs']} runs on 1 thread, "
+                      f"{c1['us_per_call']:.0f} us per call",
+            "all_cores": {"value": round(cfgs["c1"]["all_cores"]["gflops"] / 1e3, 6), "cores": ncores,
+                          "us_per_call": cfgs["c1"]["all_cores"]["us_per_call"]},
+        }
+    line["configs"] = {n: [round(r["us_per_call"], 2), round(r["roofline_frac"], 3)] if "us_per_call" in r
+                       else "error: " + r.get("error", "")[:40] for n, r in results.items()}
+    return line
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -452,6 +503,7 @@ def main():
     ap.add_argument("--no-cpu", action="store_true", help="skip the host baseline")
     ap.add_argument("--no-hot", action="store_true", help="skip the one-set (cache-hot) timing")
     ap.add_argument("--no-dist", action="store_true", help="skip the per-call distribution")
+    ap.add_argument("--details", default="", help="file for everything measured (JSON)")
     ap.add_argument("--copy-mb", type=int, default=0,
                     help="also run one plain device copy of this many MiB (counter calibration)")
     args = ap.parse_args()
@@ -529,48 +581,11 @@ def main():
         torch.cuda.synchronize()
         del src, dst
 
-    head = results.get("c1", {})
-    line = {
-        "metric": METRIC,
-        "value": head.get("tflops"),
-        "unit": "TFLOP/s",
-        "n_gpus": 1,
-        "steps": args.steps,
-        "warmup": args.warmup,
-        "ms_per_step": round(head["us_per_call"] / 1e3, 6) if "us_per_call" in head else None,
-        "higher_is_better": True,
-        "scaling": "weak",
-        "vs_baseline": None,
-        "dtype": "fp32",
-        "data": "synthetic N(0,1) Q/K/V resident in HBM (planar [3][B*S][E] buffer, seeded; calls rotate "
-                "over buffer sets totalling >= 1 GiB so operands come from HBM, not the Infinity Cache)",
-        "config": {"workload": "c1: causal self-attention forward, fp32, B=32 H=8 S=256 D=32 (E=256), "
-                               "no probs output", "B": 32, "H": 8, "S": 256, "D": 32,
-                   "parallelism": "single GPU"},
-    }
-    if "us_per_call" in head:
-        flops, _ = work(CONFIGS["c1"])
-        ach = flops / (head["us_per_call"] * 1e-6)
-        line["roofline"] = {
-            "bound": "mfma", "achieved": round(ach / 1e12, 3), "peak": PEAK_F32_MFMA / 1e12,
-            "unit": "TFLOP/s", "frac": round(ach / PEAK_F32_MFMA, 4), "traffic": read_traffic("c1"),
-        }
-    if not args.no_cpu:
-        info, ncores, cfgs = cpu_baseline()
-        c1 = cfgs["c1"]["one_thread"]
-        line["cpu_baseline"] = {
-            "value": round(c1["gflops"] / 1e3, 6), "unit": "TFLOP/s", "cores": 1, "kind": "port",
-            "sample": f"c1 (causal) through the oracle's scalar restatement of flash_attention_kernel<32>: "
-                      f"{c1['pairs']} of {c1['of_pairs']} (b,h) pairs, median of {c1['runs']} runs on 1 thread, "
-                      f"{c1['us_per_call']:.0f} us per c1 call; c2..c5 in 'configs' (subsampled pairs scaled "
-                      f"by B*H/pairs; c3/c4/c5 the fallback's 3-pass math)",
-            "host": info,
-            "all_cores": {"value": round(cfgs["c1"]["all_cores"]["gflops"] / 1e3, 6), "cores": ncores,
-                          "us_per_call": cfgs["c1"]["all_cores"]["us_per_call"]},
-            "configs": cfgs,
-        }
-    line["configs"] = results
-    print(json.dumps(line), flush=True)
+    cpu = None if args.no_cpu else cpu_baseline()
+    if args.details:
+        with open(args.details, "w") as f:
+            json.dump({"configs": results, "cpu_baseline": cpu and {"host": cpu[0], "configs": cpu[2]}}, f, indent=1)
+    print(json.dumps(headline(args.steps, args.warmup, results, cpu)), flush=True)
 
 
 if __name__ == "__main__":

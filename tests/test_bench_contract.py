@@ -83,3 +83,21 @@ def test_cpu_baseline_leg_times_the_oracle():
     r = bench.cpu_config("c1", 1, 0.05)  # at least one (b, h) pair, scaled to the whole problem
     assert r["threads"] == 1 and 1 <= r["pairs"] <= r["of_pairs"] == 256
     assert r["us_per_call"] > 0 and r["gflops"] > 0
+
+
+def test_headline_is_one_short_line():
+    # readers keep only the last few KB of stdout, so the line has to fit whole
+    full = {"us_per_call": 123456.789, "roofline_frac": 0.12345, "tflops": 1234.567}
+    results = {n: dict(full) for n in bench.CONFIGS}
+    results["c2"] = {"error": "x" * 500}
+    one = {"us_per_call": 36637456.7, "gflops": 12345.678, "threads": 16, "pairs": 256, "of_pairs": 256, "runs": 99}
+    cpu = ({}, 16, {n: {"one_thread": one, "all_cores": one} for n in bench.CPU_CONFIGS})
+    text = json.dumps(bench.headline(20, 5, results, cpu))
+    assert len(text) < 4096 and "\n" not in text
+    line = json.loads(text)
+    for key in ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "higher_is_better", "scaling",
+                "vs_baseline", "dtype", "data", "config"):
+        assert key in line
+    assert {"model", "global_batch", "seq_len", "parallelism"} <= set(line["config"])
+    assert line["value"] == 1234.567 and line["ms_per_step"] == 123.456789
+    assert set(line["configs"]) == set(bench.CONFIGS)
