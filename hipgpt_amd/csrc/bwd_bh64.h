@@ -217,53 +217,6 @@ __global__ __launch_bounds__(NW * 64) void bwd_bh64_kernel(BwdArgs a) {
         }
     }
 
-    // A chain over the head dim: acc[m = row c of `rt`][n = key c] += sum_d
-    // rt[c][d] bv[d], lane (c, h) taking d = 32h .. 32h+31 (16 at a time).
-    auto chain = [&](const float* rt, const float (&bv)[DK / 2], floatx16 acc) {
-        const float* rr = rt + c * RPd + hf * (DK / 2);
-#pragma unroll
-        for (int hb = 0; hb < DK / 32; ++hb) {
-            floatx4 dv[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) dv[j] = *reinterpret_cast<const floatx4*>(rr + 16 * hb + 4 * j);
-#pragma unroll
-            for (int k = 0; k < 16; ++k) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(dv[k >> 2][k & 3], bv[16 * hb + k], acc, 0, 0, 0);
-        }
-        return acc;
-    };
-    // dV^T += dO^T P: A[d][query] read from the row-major dO tile
-    auto grad_v = [&](const float* gt, const floatx16& pv) {
-#pragma unroll
-        for (int n = 0; n < NB; ++n)
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-                accv[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(gt[acc_key(r, hf) * RPd + 32 * n + c], pv[r], accv[n], 0, 0, 0);
-    };
-    // dK^T += Q^T dS, then the dQ term dS K: dS^T through the scratch
-    // ([key][query]), one 32-dim block at a time, each stored as it completes
-    // (register r <-> query acc_key(r, h), lane <-> dim 32n + c)
-    auto grad_kq = [&](const float* qt, const floatx16& ds) {
-#pragma unroll
-        for (int n = 0; n < NB; ++n)
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-                acck[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(qt[acc_key(r, hf) * RPd + 32 * n + c], ds[r], acck[n], 0, 0, 0);
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-            *reinterpret_cast<floatx4*>(X + c * XP + 8 * g + 4 * hf) = floatx4{ds[4 * g], ds[4 * g + 1], ds[4 * g + 2], ds[4 * g + 3]};
-        asm volatile("" ::: "memory");
-#pragma unroll
-        for (int n = 0; n < NB; ++n) {
-            floatx16 aq = __builtin_amdgcn_mfma_f32_32x32x2f32(X[dq_key(0, hf) * XP + c], kq[n][0], floatx16{}, 0, 0, 0);
-#pragma unroll
-            for (int s = 1; s < 16; ++s)
-                aq = __builtin_amdgcn_mfma_f32_32x32x2f32(X[dq_key(s, hf) * XP + c], kq[n][s], aq, 0, 0, 0);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) dqw[(8 * (r >> 2) + (r & 3)) * PPd + 32 * n] = aq[r];
-        }
-    };
-    const bool kedge = wave * BK + BK > S;  // keys past S in this wave's tile
-
     // Step t (t % 2 == PAR) of every wave.  Stored probs: pc holds P of tile
     // t, the other buffer P of tile t+1 (requested a step ago); P of tile t+2
     // goes into pc once dS is formed, so the two buffers alternate roles and
@@ -290,8 +243,6 @@ __global__ __launch_bounds__(NW * 64) void bwd_bh64_kernel(BwdArgs a) {
             for (int v = 0; v < NW; ++v) dsum += pdl[(PAR * NW + v) * BK];
             if (hf == 0) X[(c >> 2) * XP + DQCOL + (c & 3)] = dsum;
             asm volatile("" ::: "memory");
-            // (written out here: through grad_v and grad_kq this branch
-            // spills two registers at 256 VGPRs)
 #pragma unroll
             for (int n = 0; n < NB; ++n)
 #pragma unroll

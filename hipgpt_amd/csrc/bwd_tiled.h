@@ -1,25 +1,23 @@
 // bwd_tiled.h -- LDS-tiled MFMA kernels of the attention backward on the
 // forward's probabilities (HipGPT src/hip_kernels.cpp:1159-1272), for head
 // dims 32 and 64 with 16-byte aligned rows.  The workgroups of bwd_terms.h run
-// them where their split operands do not hold the data.
+// them where a result on bf16 terms is not finite.
 //
 // Math per (b, h), scale c = 1/sqrt(D):
 //   dP = dO V^T,  Dq_i = sum_j P_ij dP_ij,  dS = P o (dP - Dq),
 //   dQ = c dS K,  dK = c dS^T Q,  dV = P^T dO.
 // Two kernels, every gradient element written once (no atomics, no memset):
-//   * BwdQ (query-stationary): wave (qs, ks) owns 32 queries and every
-//     NKS-th key tile.  One pass over the keys accumulates
+//   * BwdQ (query-stationary): a wave owns 32 queries.  One pass over the keys
+//     accumulates
 //       A = (P o dP) K,  Bm = P K,  Dq = rowsum(P o dP),
-//     and dQ = c (A - Dq Bm), so P and V are read once; the key splits are
-//     summed through LDS.  Dq goes to the workspace for the second kernel.
-//   * BwdKV (key-stationary): wave (ks, qs) owns 32 keys (V in
-//     registers) and every NQS-th query tile; dP = dO V^T lands with one key
-//     per lane and the queries in the accumulator's register order, which is
-//     the B-operand layout of dV^T += dO^T P and dK^T += Q^T dS, so P and dS
-//     never leave registers; the query splits are summed through LDS.
+//     and dQ = c (A - Dq Bm), so P and V are read once.  Dq goes to the
+//     workspace for the second kernel.
+//   * BwdKV (key-stationary): a wave owns 32 keys (V in registers); dP = dO V^T
+//     lands with one key per lane and the queries in the accumulator's register
+//     order, which is the B-operand layout of dV^T += dO^T P and dK^T += Q^T dS,
+//     so P and dS never leave registers.
 // Operand tiles go global -> registers -> LDS, double buffered, one barrier
-// per stage (one key tile, resp. NQS query tiles), with the next stage's
-// loads in flight during the MFMAs.  LDS tiles are row-major (pitch DP+4:
+// per tile, with the next tile's loads in flight during the MFMAs.  LDS tiles are row-major (pitch DP+4:
 // conflict-free ds_read_b128 along the head dim) or transposed (pitch 36:
 // ds_read_b128 along the 32 rows).  P is read straight from global memory in
 // the layout each kernel needs: rows of 16 bytes (query-stationary) or
@@ -113,20 +111,18 @@ __device__ __forceinline__ int role_of(int sr, int rank, int nranks, int nw, boo
 }
 
 // ----------------------------------------------------------------- dQ, Dq
-template <int DP, int NQS, int NKS, bool CAUSAL, bool RECOMP>
+template <int DP, int NQS, bool CAUSAL, bool RECOMP>
 struct BwdQ {
     using T = Tiles<DP>;
-    static constexpr int NW = NQS * NKS;
+    static constexpr int NW = NQS;
     static constexpr int NT = NW * 64;
     static constexpr int NDB = DP / 32;
     static constexpr int NACC = RECOMP ? 1 : 2;  // accumulators: A (, Bm)
-    // stage: NKS key tiles, each V row-major + K transposed (+ K row-major,
-    // the A operand of S^T = K Q^T, when P is recomputed)
-    static constexpr int KT = T::ROW + T::TR + (RECOMP ? T::ROW : 0);
-    static constexpr int STAGE = NKS * KT;
-    static constexpr int PER = (2 * NKS * T::CPT + NT - 1) / NT;  // chunks per thread per stage
-    static constexpr int MERGE = NKS > 1 ? NW * 64 * (2 * 16 * NDB + 1) : 0;
-    static constexpr int LDS_FLOATS = 2 * STAGE > MERGE ? 2 * STAGE : MERGE;
+    // stage: a key tile, V row-major + K transposed (+ K row-major, the A operand
+    // of S^T = K Q^T, when P is recomputed)
+    static constexpr int STAGE = T::ROW + T::TR + (RECOMP ? T::ROW : 0);
+    static constexpr int PER = (2 * T::CPT + NT - 1) / NT;  // chunks per thread per stage
+    static constexpr int LDS_FLOATS = 2 * STAGE;
 
     // Workgroup `rank` of the nqb query blocks of problem bh.
     __device__ __forceinline__ static void run(const BwdArgs& a, float* lds, int* simd_slots, int nqb, int bh, int rank) {
@@ -136,8 +132,7 @@ struct BwdQ {
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
         const int c = lane & 31, hf = lane >> 5;
         const int qb = CAUSAL ? nqb - 1 - rank : rank;
-        const int role = role_of(fa::simd_rank<NW>(simd_slots, wave, lane), rank, nqb, NW, CAUSAL);
-        const int qs = role / NKS, ks = role % NKS;
+        const int qs = role_of(fa::simd_rank<NW>(simd_slots, wave, lane), rank, nqb, NW, CAUSAL);
         const int b = bh / a.H, h = bh % a.H;
         const int S = a.S;
         const int q0 = qb * NQS * BK, qw0 = q0 + qs * BK, qi = qw0 + c;
@@ -145,7 +140,6 @@ struct BwdQ {
         const int kend = CAUSAL ? min(S, q0 + NQS * BK) : S;
         const int ntiles = (kend + BK - 1) / BK;
         const int wtiles = qw0 < S ? (CAUSAL ? (min(S, qw0 + BK) + BK - 1) / BK : ntiles) : 0;
-        const int nstages = (ntiles + NKS - 1) / NKS;
 
         // dO (B operand of dP^T = V dO^T): lane (c, h) holds dO[qi][h*DP/2 + s]
         float go[DP / 2];
@@ -185,16 +179,16 @@ struct BwdQ {
         kl.init(a.k + base, a.ts, S, a.D);
         vl.init(a.v + base, a.ts, S, a.D);
         floatx4 stg[PER];
-        static_assert((NKS * T::CPT) % 64 == 0, "a wave's chunks are all K or all V");
+        static_assert((T::CPT) % 64 == 0, "a wave's chunks are all K or all V");
         auto load = [&](int st) {
 #pragma unroll
             for (int i = 0; i < PER; ++i) {
                 const int f = tid + i * NT;
-                if ((2 * NKS * T::CPT) % NT != 0 && f >= 2 * NKS * T::CPT) break;
-                const int isk = f >= NKS * T::CPT;
-                const int g = isk ? f - NKS * T::CPT : f;
-                const int row = st * NKS * BK + g / T::CPR;
-                // K or V is wave-uniform (NKS * CPT is a multiple of 64): a scalar
+                if ((2 * T::CPT) % NT != 0 && f >= 2 * T::CPT) break;
+                const int isk = f >= T::CPT;
+                const int g = isk ? f - T::CPT : f;
+                const int row = st * BK + g / T::CPR;
+                // K or V is wave-uniform (CPT is a multiple of 64): a scalar
                 // branch instead of a per-lane select of two buffer resources
                 if (__builtin_amdgcn_readfirstlane(isk))
                     stg[i] = kl.load(row, g % T::CPR);
@@ -206,16 +200,15 @@ struct BwdQ {
 #pragma unroll
             for (int i = 0; i < PER; ++i) {
                 const int f = tid + i * NT;
-                if ((2 * NKS * T::CPT) % NT != 0 && f >= 2 * NKS * T::CPT) break;
-                const int isk = f >= NKS * T::CPT;
-                const int g = isk ? f - NKS * T::CPT : f;
-                const int kt = g / T::CPT, r = (g % T::CPT) / T::CPR, cc = g % T::CPR;
-                float* tile = dst + kt * KT;
+                if ((2 * T::CPT) % NT != 0 && f >= 2 * T::CPT) break;
+                const int isk = f >= T::CPT;
+                const int g = isk ? f - T::CPT : f;
+                const int r = g / T::CPR, cc = g % T::CPR;
                 if (isk) {
-                    T::store_tr(tile + T::ROW, r, cc, stg[i]);
-                    if (RECOMP) T::store_row(tile + T::ROW + T::TR, r, cc, stg[i]);
+                    T::store_tr(dst + T::ROW, r, cc, stg[i]);
+                    if (RECOMP) T::store_row(dst + T::ROW + T::TR, r, cc, stg[i]);
                 } else {
-                    T::store_row(tile, r, cc, stg[i]);
+                    T::store_row(dst, r, cc, stg[i]);
                 }
             }
         };
@@ -247,12 +240,10 @@ struct BwdQ {
         };
         // The next tile's P is requested while this tile's MFMAs run.
         floatx4 pnext[4];
-        if (!RECOMP && ks < wtiles) load_p(pnext, ks);
+        if (!RECOMP && wtiles > 0) load_p(pnext, 0);
 
-        auto compute = [&](int st, const float* cur) {
-            const int t = st * NKS + ks;
+        auto compute = [&](int t, const float* tile) {
             if (t >= wtiles) return;
-            const float* tile = cur + ks * KT;
             floatx16 x[2];
             if constexpr (RECOMP) {
                 floatx16 sc;
@@ -272,7 +263,7 @@ struct BwdQ {
                 for (int g = 0; g < 4; ++g)
 #pragma unroll
                     for (int j = 0; j < 4; ++j) x[1][4 * g + j] = pnext[g][j];
-                if (t + NKS < wtiles) load_p(pnext, t + NKS);
+                if (t + 1 < wtiles) load_p(pnext, t + 1);
             }
             floatx16 dp;
 #pragma unroll
@@ -294,47 +285,19 @@ struct BwdQ {
             }
         };
 
-        if (nstages > 0) {
+        if (ntiles > 0) {
             load(0);
             store(lds);
         }
         __syncthreads();
-        for (int st = 0; st < nstages; ++st) {
-            if (st + 1 < nstages) load(st + 1);
+        for (int st = 0; st < ntiles; ++st) {
+            if (st + 1 < ntiles) load(st + 1);
             compute(st, lds + (st & 1) * STAGE);
-            if (st + 1 < nstages) store(lds + ((st + 1) & 1) * STAGE);
+            if (st + 1 < ntiles) store(lds + ((st + 1) & 1) * STAGE);
             __syncthreads();
         }
 
-        // sum the key splits (wave ks == 0 keeps the sub-block)
-        if (NKS > 1) {
-            float* const mo = lds;  // [NW][2*16*NDB + 1][64]
-            constexpr int W = 2 * 16 * NDB + 1;
-            if (ks != 0) {
-#pragma unroll
-                for (int n = 0; n < NACC; ++n)
-#pragma unroll
-                    for (int db = 0; db < NDB; ++db)
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) mo[(role * W + (n * NDB + db) * 16 + r) * 64 + lane] = acc[n][db][r];
-                mo[(role * W + W - 1) * 64 + lane] = ld;
-            }
-            __syncthreads();
-            if (ks == 0) {
-#pragma unroll
-                for (int j = 1; j < NKS; ++j) {
-#pragma unroll
-                    for (int n = 0; n < NACC; ++n)
-#pragma unroll
-                        for (int db = 0; db < NDB; ++db)
-#pragma unroll
-                            for (int r = 0; r < 16; ++r)
-                                acc[n][db][r] += mo[((role + j) * W + (n * NDB + db) * 16 + r) * 64 + lane];
-                    ld += mo[((role + j) * W + W - 1) * 64 + lane];
-                }
-            }
-        }
-        if (ks == 0 && qi < S) {
+        if (qi < S) {
             const float dq = RECOMP ? dqv : halves_sum(ld);
             if (!RECOMP && hf == 0) a.dvec[(int64_t)bh * S + qi] = dq;
             float* out = a.dq + base + (int64_t)qi * a.ts;
@@ -354,27 +317,24 @@ struct BwdQ {
 };
 
 // ----------------------------------------------------------------- dK, dV
-template <int DP, int NKB, int NQS, bool CAUSAL, bool RECOMP>
+template <int DP, int NKB, bool CAUSAL, bool RECOMP>
 struct BwdKV {
     using T = Tiles<DP>;
-    static constexpr int NW = NKB * NQS;
+    static constexpr int NW = NKB;
     static constexpr int NT = NW * 64;
     static constexpr int NDB = DP / 32;
-    // stage: NQS query tiles, each dO row-major + dO transposed + Q transposed
-    // + Dq (+ lse' + Q row-major, the A operand of S' = Q K^T, when P is
+    // stage: a query tile, dO row-major + dO transposed + Q transposed + Dq (+ lse' + Q row-major, the A operand of S' = Q K^T, when P is
     // recomputed)
     static constexpr int DQ_OFF = T::ROW + 2 * T::TR;
     static constexpr int LSE_OFF = DQ_OFF + BK;
     static constexpr int QROW_OFF = LSE_OFF + BK;
-    static constexpr int QT = DQ_OFF + BK + (RECOMP ? BK + T::ROW : 0);
-    static constexpr int STAGE = NQS * QT;
-    static constexpr int PER = (2 * NQS * T::CPT + NT - 1) / NT;
-    static constexpr int MERGE = NQS > 1 ? NW * 64 * (2 * 16 * NDB) : 0;
-    static constexpr int LDS_FLOATS = 2 * STAGE > MERGE ? 2 * STAGE : MERGE;
+    static constexpr int STAGE = DQ_OFF + BK + (RECOMP ? BK + T::ROW : 0);
+    static constexpr int PER = (2 * T::CPT + NT - 1) / NT;
+    static constexpr int LDS_FLOATS = 2 * STAGE;
     // Recompute mode forms Dq from the staged dO chunks: chunks i < NG of a
     // thread are dO, and a row's CPR chunks sit in consecutive lanes.
-    static constexpr int NG = NQS * T::CPT / NT;
-    static_assert(!RECOMP || (NQS * T::CPT) % NT == 0, "dO chunks must fill whole passes");
+    static constexpr int NG = T::CPT / NT;
+    static_assert(!RECOMP || (T::CPT) % NT == 0, "dO chunks must fill whole passes");
 
     // Workgroup `rank` (the key block) of the nkb key blocks of problem bh.
     __device__ __forceinline__ static void run(const BwdArgs& a, float* lds, int* simd_slots, int nkb, int bh, int rank) {
@@ -384,8 +344,7 @@ struct BwdKV {
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
         const int c = lane & 31, hf = lane >> 5;
         const int kb = rank;  // key block; causal: block 0 sees the most query tiles and launches first
-        const int role = role_of(fa::simd_rank<NW>(simd_slots, wave, lane), rank, nkb, NW, CAUSAL);
-        const int ksub = role / NQS, qsp = role % NQS;
+        const int ksub = role_of(fa::simd_rank<NW>(simd_slots, wave, lane), rank, nkb, NW, CAUSAL);
         const int b = bh / a.H, h = bh % a.H;
         const int S = a.S;
         const int k0 = kb * NKB * BK, kw0 = k0 + ksub * BK, kj = kw0 + c;
@@ -394,7 +353,7 @@ struct BwdKV {
         // query tiles [it0, nq): causal starts at the workgroup's first key tile
         const int it0 = CAUSAL ? k0 / BK : 0;
         const int wit0 = CAUSAL ? kw0 / BK : 0;  // this wave's first useful query tile
-        const int nstages = (nq - it0 + NQS - 1) / NQS;
+        const int nstages = nq - it0;
 
         // V (B operand of dP = dO V^T): lane (c, h) holds V[kj][h*DP/2 + s]
         float vr[DP / 2];
@@ -427,15 +386,15 @@ struct BwdKV {
         floatx4 ostg[RECOMP ? NG : 1];  // O chunks matching the dO chunks (recompute mode)
         float dqs = 0.f;   // Dq value this thread stages (stored-probs mode)
         float lses = 0.f;  // lse' value this thread stages (+inf past the last row: P = 0)
-        static_assert((NQS * T::CPT) % 64 == 0, "a wave's chunks are all Q or all dO");
+        static_assert((T::CPT) % 64 == 0, "a wave's chunks are all Q or all dO");
         auto load = [&](int st) {
-            const int qt0 = it0 + st * NQS;
+            const int qt0 = it0 + st;
 #pragma unroll
             for (int i = 0; i < PER; ++i) {
                 const int f = tid + i * NT;
-                if ((2 * NQS * T::CPT) % NT != 0 && f >= 2 * NQS * T::CPT) break;
-                const int isq = f >= NQS * T::CPT;
-                const int g = isq ? f - NQS * T::CPT : f;
+                if ((2 * T::CPT) % NT != 0 && f >= 2 * T::CPT) break;
+                const int isq = f >= T::CPT;
+                const int g = isq ? f - T::CPT : f;
                 const int row = qt0 * BK + g / T::CPR;
                 if (__builtin_amdgcn_readfirstlane(isq))  // wave-uniform, as above
                     stg[i] = ql.load(row, g % T::CPR);
@@ -445,7 +404,7 @@ struct BwdKV {
                     if (i < NG) ostg[i] = ol.load(row, g % T::CPR);
                 }
             }
-            if (tid < NQS * BK) {
+            if (tid < BK) {
                 const int qrow = qt0 * BK + tid;
                 if (RECOMP)
                     lses = qrow < S ? a.lse[(int64_t)bh * S + qrow] * kLog2e : kInf;
@@ -457,17 +416,16 @@ struct BwdKV {
 #pragma unroll
             for (int i = 0; i < PER; ++i) {
                 const int f = tid + i * NT;
-                if ((2 * NQS * T::CPT) % NT != 0 && f >= 2 * NQS * T::CPT) break;
-                const int isq = f >= NQS * T::CPT;
-                const int g = isq ? f - NQS * T::CPT : f;
-                const int qt = g / T::CPT, r = (g % T::CPT) / T::CPR, cc = g % T::CPR;
-                float* tile = dst + qt * QT;
+                if ((2 * T::CPT) % NT != 0 && f >= 2 * T::CPT) break;
+                const int isq = f >= T::CPT;
+                const int g = isq ? f - T::CPT : f;
+                const int r = g / T::CPR, cc = g % T::CPR;
                 if (isq) {
-                    T::store_tr(tile + T::ROW + T::TR, r, cc, stg[i]);
-                    if (RECOMP) T::store_row(tile + QROW_OFF, r, cc, stg[i]);
+                    T::store_tr(dst + T::ROW + T::TR, r, cc, stg[i]);
+                    if (RECOMP) T::store_row(dst + QROW_OFF, r, cc, stg[i]);
                 } else {
-                    T::store_row(tile, r, cc, stg[i]);
-                    T::store_tr(tile + T::ROW, r, cc, stg[i]);
+                    T::store_row(dst, r, cc, stg[i]);
+                    T::store_tr(dst + T::ROW, r, cc, stg[i]);
                 }
                 if constexpr (RECOMP) {
                     // Dq of row r: the chunk dots summed over the row's CPR lanes
@@ -478,15 +436,15 @@ struct BwdKV {
                         for (int j = 1; j < 4; ++j) d = fmaf(stg[i][j], ostg[i][j], d);
 #pragma unroll
                         for (int m = 1; m < T::CPR; m <<= 1) d += __shfl_xor(d, m);
-                        if (cc == 0) tile[DQ_OFF + r] = d;
+                        if (cc == 0) dst[DQ_OFF + r] = d;
                     }
                 }
             }
-            if (tid < NQS * BK) {
+            if (tid < BK) {
                 if (RECOMP)
-                    dst[(tid / BK) * QT + LSE_OFF + tid % BK] = lses;
+                    dst[LSE_OFF + tid] = lses;
                 else
-                    dst[(tid / BK) * QT + DQ_OFF + tid % BK] = dqs;
+                    dst[DQ_OFF + tid] = dqs;
             }
         };
 
@@ -507,19 +465,13 @@ struct BwdKV {
                 pv[r] = (qr < S && kj < S) ? pcol[(int64_t)qr * S] : 0.f;
             }
         };
-        // The wave's tiles are it = it0 + st*NQS + qsp for st = 0, 1, ...;
-        // the next one's P is requested while this one's MFMAs run.
+        // The next tile's P is requested while this one's MFMAs run.
         floatx16 pnext;
-        if (!RECOMP) {
-            int it = it0 + qsp;
-            while (it < wit0) it += NQS;
-            if (it < nq) load_p(pnext, it);
-        }
+        if (!RECOMP && wit0 < nq) load_p(pnext, wit0);
 
-        auto compute = [&](int st, const float* cur) {
-            const int it = it0 + st * NQS + qsp;
-            if (it >= nq || it < wit0) return;
-            const float* tile = cur + qsp * QT;
+        auto compute = [&](int st, const float* tile) {
+            const int it = it0 + st;
+            if (it < wit0) return;
             floatx16 x[2];  // [0] = P, [1] = dS, register r <-> query it*32 + acc_key(r, h)
             if constexpr (RECOMP) {
                 floatx16 sc;
@@ -540,7 +492,7 @@ struct BwdKV {
                 }
             } else {
                 x[0] = pnext;
-                if (it + NQS < nq) load_p(pnext, it + NQS);
+                if (it + 1 < nq) load_p(pnext, it + 1);
             }
             floatx16 dp;
 #pragma unroll
@@ -570,31 +522,7 @@ struct BwdKV {
             __syncthreads();
         }
 
-        if (NQS > 1) {
-            float* const mo = lds;  // [NW][2*16*NDB][64]
-            constexpr int W = 2 * 16 * NDB;
-            if (qsp != 0) {
-#pragma unroll
-                for (int n = 0; n < 2; ++n)
-#pragma unroll
-                    for (int db = 0; db < NDB; ++db)
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) mo[(role * W + (n * NDB + db) * 16 + r) * 64 + lane] = acc[n][db][r];
-            }
-            __syncthreads();
-            if (qsp == 0) {
-#pragma unroll
-                for (int j = 1; j < NQS; ++j)
-#pragma unroll
-                    for (int n = 0; n < 2; ++n)
-#pragma unroll
-                        for (int db = 0; db < NDB; ++db)
-#pragma unroll
-                            for (int r = 0; r < 16; ++r)
-                                acc[n][db][r] += mo[((role + j) * W + (n * NDB + db) * 16 + r) * 64 + lane];
-            }
-        }
-        if (qsp == 0 && kj < S) {
+        if (kj < S) {
             float* dvp = a.dv + base + (int64_t)kj * a.ts;
             float* dkp = a.dk + base + (int64_t)kj * a.ts;
 #pragma unroll

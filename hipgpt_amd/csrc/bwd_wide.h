@@ -4,8 +4,8 @@
 // and 256 (whose per-wave accumulators and dO / V rows would not fit one
 // wave's registers) and head dims below 64 that are not 32 or 64, any D with
 // D % 4 == 0 and 16-byte aligned rows.  Head dims above 128 run them as
-// kernels; below, the workgroups of bwd_terms.h where their split operands do
-// not hold the data.
+// kernels; below, the workgroups of bwd_terms.h where a result on bf16 terms is
+// not finite.
 //
 // Same math and the same two kernels as bwd_tiled.h (query-stationary dQ and
 // row dots Dq through A = (P o dP) K and Bm = P K; key-stationary dK, dV with

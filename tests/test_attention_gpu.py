@@ -93,13 +93,12 @@ def test_small_grid_key_split_matches_oracle(dev, B, S, E, H, causal, with_probs
         assert np.abs(host(d_p) - want_p).max() <= TOL_P
 
 
-# D = 64 with probs, 193 <= S <= 256 and B*H at least the CU count (256 on
-# MI355X): the one-workgroup-per-(b, h) resident kernel, at ragged S; the
-# same shapes without probs run the streaming kernel.
+# D = 64 with B*H at least the CU count (256 on MI355X), at ragged S of up to 256
+# keys: full grids of short rows, with probs and without.
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("with_probs", [True, False])
 @pytest.mark.parametrize("B,S,E,H", [(32, 200, 512, 8), (64, 250, 256, 4)])
-def test_resident_kernel_matches_oracle(dev, B, S, E, H, causal, with_probs):
+def test_full_grid_short_rows_match_oracle(dev, B, S, E, H, causal, with_probs):
     qkv = O.seeded_planar(S * 19 + E + B, B, S, E)
     want_o, want_p = O.launch_multihead_attention(qkv, B, S, E, H, causal=causal, want_probs=True)
     d_out = torch.full((B * S, E), float("nan"), device=dev)

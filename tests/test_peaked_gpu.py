@@ -5,12 +5,10 @@ argmax limit (Q scaled by 1e4).
 These inputs make the online softmax move its running max far and often
 (the lazy rescale, which only rescales O once a row max grows by more than
 2^8), and they run the score-resident, recomputed and spilled probs sweeps
-and the resident-K/V kernel with scores far from the unit-variance range.
+with scores far from the unit-variance range.
 
 Shapes: c1 (D=32, streaming kernel, scores kept in registers with probs),
-c2 (D=64, S=256, B*H=256: the resident-K/V kernel with probs, the streaming
-kernel without), c3 (D=64, S=1024:
-streaming 4x2, Q.K^T recomputed with probs) and c4's head shape at B=1
+c2 (D=64, S=256, B*H=256), c3 (D=64, S=1024: Q.K^T recomputed with probs) and c4's head shape at B=1
 (D=128, S=2048: probs rows spilled and read back).
 
 Bars.  fp32 rounding of a score s costs about eps*|s|, and |s| grows with the
