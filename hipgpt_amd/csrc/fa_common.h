@@ -146,7 +146,7 @@ __device__ __forceinline__ void store_probs_tile(float* prow, const floatx16& p,
 
 // Causal: zero the probs of this wave's queries for keys >= z0 (whole rows
 // per instruction; non-temporal if NT: the score-resident streaming sweep,
-// c1 with probs 27.7 -> 26.6 us; the other probs paths measured 1-9% slower
+// on fp32 MFMA B32 H8 S256 D32 with probs 27.7 -> 26.6 us; the other probs paths measured 1-9% slower
 // with it).
 template <bool NT = false>
 __device__ __forceinline__ void zero_probs_tail(float* probs_bh, int qw0, int Sq, int Sk, int z0, int lane, bool pvec) {

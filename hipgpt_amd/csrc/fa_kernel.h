@@ -34,30 +34,20 @@ namespace fa {
 // Start stagger of short causal grids (see FaKernel::run): 35 ticks of the
 // 100 MHz s_memrealtime counter = 350 ns per launch rank, for grids of at
 // most 4 query blocks per (batch, head) that are resident at once and fill
-// at least half of the device's workgroup slots (c1: 16.1 -> 15.8 us against 200 ns;
-// measured over 100 .. 800 ns per rank; re-measured on cache-rotated inputs
-// at 250 .. 550 ns: within 0.1 us rotated, 350 ns best hot).
+// at least half of the device's workgroup slots.  Cache-rotated, interleaved,
+// us without and with: B16 H8 S512 D32 causal 22.3, 21.7; D64 38.3, 37.8; two
+// query blocks (B32 H8 S256) level.
 constexpr unsigned long long kStaggerTicks = 35;
-// The same for grids that write probs: 1 us per rank without a causal mask
-// (c1 drop-in 31.3 -> 29.9 us), 700 ns with one (c1 with probs 25.0 ->
-// 24.7 us); measured over 0.4 .. 1.6 us per rank.
+// The same for grids that write probs: 1 us per rank without a causal mask (B16
+// H8 S512 D32 59.0 -> 58.2, B32 H8 S256 D64 45.8 -> 45.3), 700 ns with one (B16
+// H8 S512 D32 50.0 -> 49.3, B32 H8 S256 D64 37.8 -> 37.2).
 constexpr unsigned long long kStaggerTicksProbs = 100;
 constexpr unsigned long long kStaggerTicksProbsCausal = 70;
-// Probs tiles of the score-resident sweep, and of the causal probs sweeps at
-// padded head dims >= kTransOwnMinDP (one workgroup per CU, LDS to spare),
-// are stored through a per-wave LDS transpose as whole 128-byte rows,
-// non-temporally, instead of straight from the accumulator layout (32 bytes
-// per row per instruction).  Measured (cache-rotated / hot, us): c1 with probs
-// 31.2 / 24.5 -> 28.6 / 24.6, the c1 drop-in 34.9 / 29.6 -> 33.1 / 30.0,
-// B = 128 drop-in 138.7 / 124.2 -> 124.7 / 111.2; plain (not non-temporal)
-// whole-row stores gained less rotated and lost hot.  The spilled scores of
-// those causal sweeps leave the same way.
-constexpr int kTransOwnMinDP = 128;
+// Probs tiles of the score-resident sweep are stored through a per-wave LDS
+// transpose as whole 128-byte rows, non-temporally, instead of straight from the
+// accumulator layout (32 bytes per row per instruction).
 // O stores of the streaming kernel go through a per-wave LDS transpose as
-// whole rows of the head, non-temporally: c1 17.85 -> 16.84 us (cache-rotated;
-// hot 15.77 -> 14.95), the c1 drop-in 33.2 -> 31.4 us; the transpose with
-// plain stores measured level, and non-temporal stores of the accumulator
-// layout's 32-byte row pieces were slower (c1 17.6 us).
+// whole rows of the head, non-temporally.
 // Start stagger only for grids of at most this many query blocks per (b, h).
 constexpr int kStaggerMaxBlocks = 4;
 
@@ -82,14 +72,8 @@ struct stage_buffers<TR, std::void_t<decltype(TR::NBUF)>> { static constexpr int
 // SRT < 0 (probs only, rows longer than that): the max/sum sweep stores each
 // masked score tile into the probs buffer, where the probs sweep reads it back
 // and overwrites it with P -- two products instead of three (no second Q K^T,
-// no K staging) for one more write and read of the probs rows.  With the
-// accumulator-layout stores each lane reads back only what it wrote, in the
-// same sweep order.  With the per-wave LDS transpose (TRANS_OWN: causal, padded
-// head dim >= 128) a tile's scores leave as whole rows, so lanes write other
-// lanes' rows and the read-back is cross-lane: it is correct only because every
-// sweep iteration ends with a workgroup barrier (and one precedes the first
-// read-back prefetch), which orders each global store before the loads of the
-// other lanes.  A change that removes those barriers breaks the spill.
+// no K staging) for one more write and read of the probs rows.  Each lane reads
+// back only what it wrote, in the same sweep order.
 template <class TR, int NQS, int NKS, bool CAUSAL, bool PROBS, bool VEC, int SRT = 0>
 struct FaKernel {
     static constexpr int DP = TR::DP;
@@ -110,31 +94,23 @@ struct FaKernel {
     static constexpr int MERGE_BYTES = NKS > 1 ? NW * 64 * (16 * NDB + 2) * 4 : 0;  // key-split merge only
     static constexpr int BASE_BYTES = (NBUF * STAGE_BYTES > MERGE_BYTES) ? NBUF * STAGE_BYTES : MERGE_BYTES;
     // Probs stores through a per-wave LDS transpose (see store_t): the score-
-    // resident sweep borrows the idle K half of the stage buffers; the causal
-    // probs sweeps at padded D >= kTransOwnMinDP (one workgroup
-    // per CU, LDS to spare) get a region of their own after BASE_BYTES, for
-    // the spilled scores and the probs alike (B4 H16 S2048 D128 with probs
-    // 880 -> 867 us).  Unmasked there, the transpose measured slower (the
-    // drop-in 1391 -> 1465 us).
+    // resident sweep borrows the idle K half of the stage buffers.
     static constexpr bool TRANS_RES =
         SRT > 0 && F32IN && TR::KTILE * (int)sizeof(E) >= QW * 36 * 4 && NW <= NBUF * NKS;
-    static constexpr bool TRANS_OWN = PROBS && CAUSAL && SRT <= 0 && F32IN && DP >= kTransOwnMinDP;
-    static constexpr int LDS_BYTES = BASE_BYTES + (TRANS_OWN ? NW * QW * 36 * 4 : 0);
+    static constexpr int LDS_BYTES = BASE_BYTES;
     // Without probs, the first stage stages K alone: the first Q K^T waits for
     // the K rows only, V of that stage is requested once K has landed and is
     // stored while the first tile's softmax runs (one more workgroup barrier).
-    // Cache-rotated: c1 (fp32, D = 32) 16.86 -> 16.62 us, c3-bf16 31.14 ->
-    // 30.38 us; fp32 D = 64 (c3) 128.3 -> 128.8 us and D = 128 (c4) level, so
-    // those keep the joint first stage.
+    // Cache-rotated, us without and with: fp32 D = 32 causal B64 H8 S256 24.8, 23.3,
+    // B8 H8 S1024 40.0, 38.0; fp32 D = 64 level (B8 H12 S1024 87.5, 87.1), which keeps
+    // the joint first stage; bf16 B8 H12 S1024 D64 31.1, 30.4.
     static constexpr bool K_FIRST = !PROBS && (!F32IN || DP == 32);
     // Online-softmax sweeps with 16-byte loads test the running max through
-    // the exponentials' sum (kLazySum) after each wave's first tile.
-    // Cache-rotated, two interleaved repetitions: c1 16.63 -> 16.56 us, c3
-    // 127.9 -> 127.4, c3-bf16 29.56 -> 29.24, c4 580.2 -> 576.7; without a
-    // causal mask at the c4 shape 1077 -> 1066, at c3-bf16's 47.4 -> 47.0,
-    // the c1 and c3 shapes level; results unchanged bit for bit.  The
-    // guarded-load instances (padded head dims) spill registers with it
-    // (25 at D = 128) and keep the max test.
+    // the exponentials' sum (kLazySum) after each wave's first tile; results
+    // unchanged bit for bit.  The guarded-load instances (padded head dims) and
+    // fp32 operands at D >= 64 spill registers with it and keep the max test:
+    // causal, us with and without, B8 H12 S1024 D64 126, 87, B4 H16 S2048 D128 530,
+    // 344; D = 32 B8 H12 S1024 48.0, 48.6.
     static constexpr bool SUM_CHECK = VEC && !(TERMS && DP >= 64);
     // What O carries of the terms' scale (P and V).
     static constexpr float O_UNSCALE = TERMS ? kTermUnscale2 : 1.f;
@@ -143,11 +119,9 @@ struct FaKernel {
     // call, on Q rows nobody has read: each workgroup of rank r reads the Q
     // rows of rank r + pf_ranks (same (b, h), same XCD) once during its
     // second stage, one 4-byte load per 64 bytes of row, so those rows come
-    // from the caches when that workgroup starts.  Cache-rotated, two
-    // interleaved repetitions: c3-bf16 29.7 -> 29.1 us, bf16 B16 H12 S1024
-    // 50.0 -> 47.2, c3 127.0 -> 126.5, fp32 B16 H12 S1024 228.6 -> 226.4;
-    // fp32 D = 32 (B32 H8 S1024 155.8 -> 157.0) and D = 128 (c4 577 -> 579)
-    // measured level or slower and go without.
+    // from the caches when that workgroup starts.  Cache-rotated, bf16 D64 B8 H12
+    // S1024 29.7 -> 29.1 us, B16 50.0 -> 47.2; fp32 D64 B8 H12 S1024, new inputs each
+    // pass, 84.9 -> 83.3.
     static constexpr bool PF_LATE = CAUSAL && !PROBS && (!F32IN || DP == 64);
     // Score-resident sweeps over at most two stages at D = 32 (the small
     // problems' 1 x 4 workgroups: HipGPT's generation call): K and V of both
@@ -286,7 +260,8 @@ struct FaKernel {
             // Two waves per SIMD: the second takes the mirror (NQS-1-qs,
             // NKS-1-ks) of the first's role, so in the diagonal stages, where
             // sub-block qs stops after its own diagonal tile, the waves still
-            // busy sit on different SIMDs (c3 128.4 -> 127.1 us, c4 604 -> 586).
+            // busy sit on different SIMDs (on fp32 MFMA
+            // 604 -> 586 us at B4 H16 S2048 D128).
             const int b = ((sr >> 1) + rank) % 4;
             const int qb0 = b / NKS, kb0 = b % NKS;
             role = (sr & 1) ? (NQS - 1 - qb0) * NKS + (NKS - 1 - kb0) : qb0 * NKS + kb0;
@@ -310,7 +285,7 @@ struct FaKernel {
         // first stage at the same moment, and the first tile computes only
         // when that burst has drained.  Launch rank r waits r * 350 ns first,
         // so the longest query blocks (rank 0) get their operands earliest
-        // and compute while the shorter ones load (c1: 16.4 -> 15.9 us).
+        // and compute while the shorter ones load (kStaggerTicks).
         // Writing probs, the ranks are spread further apart, so one rank's
         // probs stores (the second sweep, HBM-bound) overlap the next rank's
         // score sweep (MFMA-bound) instead of every workgroup storing at once.
@@ -432,7 +407,6 @@ struct FaKernel {
             }
             asm volatile("" ::: "memory");  // the next tile's writes come after these reads
         };
-        float* const Xown = reinterpret_cast<float*>(lds_raw + BASE_BYTES) + wave * QW * 36;
 
         // Exponentials of a score tile with the lazy rescale: the running max is
         // raised only when a row's tile max exceeds it by more than kLazyMax.
@@ -503,10 +477,7 @@ struct FaKernel {
                 l_run += ls;  // this lane half's partial; the halves are summed after the sweep
                 TR::pv(vreg, TR::to_p(s), o, c, hf);
             } else if constexpr (MODE == 1) {
-                if constexpr (SPILL && TRANS_OWN)
-                    store_t(Xown, prow - (int64_t)c * Sk, s, t * BK, pvec);
-                else if (SPILL && qi < Sq)
-                    store_probs_tile(prow, s, t * BK, hf, Sk, pvec);
+                if (SPILL && qi < Sq) store_probs_tile(prow, s, t * BK, hf, Sk, pvec);
                 const float m_new = vmax(m_run, tile_max(s) * sc);
                 float ls = kSumInit;
 #pragma unroll
@@ -516,10 +487,7 @@ struct FaKernel {
             } else {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) s[r] = fast_exp2(fmaf(s[r], sc, -mlog));
-                if constexpr (TRANS_OWN)
-                    store_t(Xown, prow - (int64_t)c * Sk, s, t * BK, pvec);
-                else if (qi < Sq)
-                    store_probs_tile(prow, s, t * BK, hf, Sk, pvec);
+                if (qi < Sq) store_probs_tile(prow, s, t * BK, hf, Sk, pvec);
                 TR::pv(vreg, TR::to_p(s), o, c, hf);
             }
         };
@@ -747,7 +715,7 @@ struct FaKernel {
         } else {
             // Causal: the zeros above the diagonal need no data, so they are
             // stored before the sweeps, while the first stage's loads are in
-            // flight (c1 with probs 26.5 -> 25.2 us against storing them last).
+            // flight (on fp32 MFMA 26.5 -> 25.2 us at B32 H8 S256 D32 against storing them last).
             if (CAUSAL && qw0 < Sq && ks == 0) {
                 const bool pv0 = (Sk & 3) == 0 && (reinterpret_cast<uintptr_t>(a.probs) & 15) == 0;
                 zero_probs_tail<(SRT > 0)>(a.probs + (int64_t)bh * Sq * Sk, qw0, Sq, Sk, tr.wtiles * BK, lane, pv0);
@@ -932,10 +900,9 @@ hipError_t launch_fa(const AttnArgs& a, hipStream_t stream) {
     // Causal grids of more than one round of resident workgroups but under
     // two: the last whole launch rank of the first round runs the shortest
     // query block instead of the next longest, so its slots free early and
-    // the blocks of the second round start sooner.  Cache-rotated, three
-    // interleaved repetitions: c3 127.2 -> 125.5 us, c3-bf16 28.9 -> 28.8
-    // (hot 26.8 -> 26.2), c3 with probs level; grids of two whole rounds
-    // keep the plain order (c4 575 -> 632 with it).
+    // the blocks of the second round start sooner.  Cache-rotated, interleaved:
+    // bf16 B8 H12 S1024 D64 28.9 -> 28.8 us (hot 26.8 -> 26.2), fp32 there level (85.5,
+    // 85.2); grids of two whole rounds keep the plain order.
     args.short_rank = 0;
     if (CAUSAL && args.n_qblk > 2) {
         const int slots = cache.get(reinterpret_cast<const void*>(kern), NQS * NKS * 64, 0);
@@ -955,13 +922,15 @@ hipError_t launch_fa(const AttnArgs& a, hipStream_t stream) {
 }
 
 // Probs rows that do not fit the score-resident stages spill their scores to
-// the probs buffer between the sweeps (1) or recompute Q K^T (0).  Reading a
-// spilled 32x32 tile back costs 4 KB per query sub-block whatever the head
-// size; recomputing it costs a staged K tile (32 * D * 4 bytes, shared by the
-// workgroup) and 32 * 32 * D MFMA work.  The spill measured faster on fp32
-// operands at D = 128 (B4 H16 S2048: 1623 -> 1504 us for the drop-in
-// launcher) and slower at D = 64 (B8 H12 S1024: 327 -> 388 us), so it is
-// used for fp32 operands with a padded head size of 128 or more.
+// the probs buffer between the sweeps or recompute Q K^T.  Reading a spilled
+// 32x32 tile back costs 4 KB per query sub-block whatever the head size;
+// recomputing it costs a staged K tile (converted, and shared by the workgroup)
+// and 32 * 32 * D MFMA work.  fp32 operands with a padded head size of 128 or
+// more spill, except in workgroups of eight query sub-blocks, which share each K
+// tile most and run the largest grids, whose scores have left the caches by then.
+// D = 128, us, spilled and recomputed: unmasked B2 H8 S256 28.7, 33.8, B1 H8 S2048
+// 217, 235, B32 H8 S256 84, 91, B8 H8 S1024 293, 289; eight sub-blocks B16 H16
+// S512 310, 292, B8 H16 S1024 605, 551, B4 H16 S2048 1143, 1037.
 constexpr int kScoreSpillMinDP = 128;
 
 // Score-resident stages of a traits type (PROBS_RES_STAGES; 0 = the probs
@@ -973,24 +942,16 @@ struct probs_res_stages<TR, std::void_t<decltype(TR::PROBS_RES_STAGES)>> {
     static constexpr int value = TR::PROBS_RES_STAGES;
 };
 
-// Instances of one workgroup shape chosen by the runtime flags.  CAUSAL_INST
-// false: the caller launches it without a causal mask only, and no causal
-// instance is compiled.
-template <class TR, int NQS, int NKS, bool VEC, bool CAUSAL_INST = true>
+// Instances of one workgroup shape chosen by the runtime flags.
+template <class TR, int NQS, int NKS, bool VEC>
 hipError_t launch_fa_flags(const AttnArgs& a, bool causal, bool probs, hipStream_t s) {
     constexpr int SRT = probs_res_stages<TR>::value;
-    constexpr bool kSpill = VEC && sizeof(typename TR::gelem) == 4 && TR::DP >= kScoreSpillMinDP;
-    if constexpr (!CAUSAL_INST) {
-        if (causal) return hipErrorInvalidValue;
-    }
+    constexpr bool kSpill = VEC && sizeof(typename TR::gelem) == 4 && TR::DP >= kScoreSpillMinDP && NQS < 8;
     // causal and non-causal instances of one choice of PROBS and SRT
     auto by_mask = [&](auto probs_tag, auto srt_tag) -> hipError_t {
         constexpr bool P = decltype(probs_tag)::value;
         constexpr int R = decltype(srt_tag)::value;
-        if constexpr (CAUSAL_INST) {
-            if (causal) return launch_fa<TR, NQS, NKS, true, P, VEC, R>(a, s);
-        }
-        return launch_fa<TR, NQS, NKS, false, P, VEC, R>(a, s);
+        return causal ? launch_fa<TR, NQS, NKS, true, P, VEC, R>(a, s) : launch_fa<TR, NQS, NKS, false, P, VEC, R>(a, s);
     };
     using yes = std::true_type;
     using no = std::false_type;
