@@ -58,7 +58,8 @@ struct WideQ {
 
     __device__ __forceinline__ static void run(const BwdArgs& a, float* lds, int nqb, int bh, int rank) {
         int tid = threadIdx.x;
-        asm volatile("" : "+v"(tid));  // as a second pass: nothing of the first stays live for it
+        // as a second pass (head dims up to 128): nothing of the first stays live for it
+        if constexpr (DP <= 128) asm volatile("" : "+v"(tid));
         const int lane = tid & 63;
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
         const int c = lane & 31, hf = lane >> 5;
@@ -238,7 +239,8 @@ struct WideKV {
 
     __device__ __forceinline__ static void run(const BwdArgs& a, float* lds, int bh, int rank) {
         int tid = threadIdx.x;
-        asm volatile("" : "+v"(tid));  // as a second pass: nothing of the first stays live for it
+        // as a second pass (head dims up to 128): nothing of the first stays live for it
+        if constexpr (DP <= 128) asm volatile("" : "+v"(tid));
         const int lane = tid & 63;
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
         const int c = lane & 31, hf = lane >> 5;

@@ -256,15 +256,14 @@ struct F32TermTraits {
 // unless a second costs no workgroup.  SRES: probs rows of up to SRES stages
 // keep their scores in registers between the two sweeps.
 // us, shapes (x NBUF) at n128; c: causal, f: unmasked, p: unmasked with probs:
-//   D=32, 256 keys: 128 c 1x4 9.0, 2x2x2 9.5, 2x4 9.6, f 10.6, 9.2, 9.4, p 12.3,
-//     14.5, 15.6; 256 c 2x2x2 10.3, 4x2 11.4, f 12.1, 11.6, p 16.8, 20.8; 1024 c
-//     4x1x2 22.8, 4x2 25.0, 2x2x2 30.8, p 57.7, 61.1, 56.1.  1024 keys: 64 c 1x4
-//     18.1, 2x4 19.4, 2x2x2 22.5; 128 p 2x4 37.8, 1x4 45.7; 256 c 2x2x2 24.3, 2x4
+//   D=32, 256 keys: 128 c 1x4 9.0, 2x2x2 9.5, 2x4 9.6, f 10.6, 9.2, 9.4; 256 c
+//     2x2x2 10.3, 4x2 11.4, f 12.1, 11.6; 1024 c 4x1x2 22.8, 4x2 25.0, 2x2x2 30.8.
+//     1024 keys: 64 c 1x4 18.1, 2x4 19.4, 2x2x2 22.5; 128 p 2x4 37.8, 1x4 45.7; 256 c 2x2x2 24.3, 2x4
 //     25.2, 4x2 29.0, f 34.9, 37.5, 30.8, p 69.5, 59.6, 65.6; 1024 c 4x2 60.4,
 //     4x1x2 62.9, 2x2x2 71.8.
 //   D=64, 256 keys: 128 2x2 14.0, 2x4 14.1, 4x2 16.9; 256 c 2x2 14.7, 4x2 17.5, f
-//     19.9, 18.8, p 25.6, 28.9; 1024 c 4x1 42.0, 8x1 54.4, 2x2 51.7.  1024 keys:
-//     128 2x4 32.5, 2x2 38.0, 4x2 45.8; 256 c 2x2 41.4, 2x4 42.6, 4x2 46.9, f 60.2,
+//     19.9, 18.8, p 25.6, 28.9; 512 c 4x1x2 26.4, 4x1 27.8, with probs 43.8, 49.7; 1024 c
+//     4x1 42.0, 8x1 54.4, 2x2 51.7.  1024 keys: 128 2x4 32.5, 2x2 38.0, 4x2 45.8; 256 c 2x2 41.4, 2x4 42.6, 4x2 46.9, f 60.2,
 //     65.1, 52.4, p 98.6, 107.9, 92.6; 512 c 4x2 60.5, 4x1 69.3, f 104, 98.8; 768 c
 //     4x1 85.6, 4x1x2 89.3, 4x2 92.6, p 246, 264, 275.
 //   D=128, 256 keys: 128 2x2 26.4, 4x1x2 33.5; 256 2x2 38.1, 4x1x2 34.1; 512 4x1
@@ -276,17 +275,22 @@ hipError_t launch_shape(const AttnArgs& a, bool causal, bool probs, hipStream_t 
     return fa::launch_fa_flags<F32TermTraits<DP, NBUF, SRES, WPE>, NQS, NKS, VEC>(a, causal, probs, s);
 }
 
-// Small grids over rows of 129 to 256 keys on fp32 MFMA itself, two stages of a 1 x
-// 4 workgroup: each call is one short chain of load, scores, softmax and product
-// per wave, which the terms' conversion lengthens.  us, terms against this, 16
-// and 64 blocks of 128 rows: D=32 with probs 8.5, 7.6 and 8.9, 8.0, causal 7.9,
-// 7.7 and 7.9, 7.4; D=64 level (12.7, 12.8; 12.5, 12.3).
-template <int DP>
-hipError_t launch_small(const AttnArgs& a, bool causal, bool probs, hipStream_t s) {
+// Short calls on fp32 MFMA itself, rows of at most 32 NKS SRES keys (with probs
+// their scores stay in registers): in small grids each call is one short chain of
+// load, scores, softmax and product per wave, which the terms' conversion
+// lengthens, and at D = 32 with probs the stores bound the larger ones.  us, terms
+// against this, blocks of 128 rows: D=32, 256 keys, unmasked probs 16 8.5, 7.6; 128
+// 12.3, 11.7; 512 34.0, 31.5; 1024 66.1, 60.9; causal probs 512 31.1, 26.9; 1024 60.2,
+// 51.4 (without probs 22.8, 30.8); 128 keys, causal probs 1024 46.4, 38.5.  D=64, 64
+// blocks 12.5, 12.3; 128 19.8, 22.1.
+template <int DP, int NQS, int NKS, int SRES>
+hipError_t launch_f32(const AttnArgs& a, bool causal, bool probs, hipStream_t s) {
     using T = F32Traits<DP, 2>;
     if (probs)
-        return causal ? fa::launch_fa<T, 1, 4, true, true, true, 2>(a, s) : fa::launch_fa<T, 1, 4, false, true, true, 2>(a, s);
-    return causal ? fa::launch_fa<T, 1, 4, true, false, true>(a, s) : fa::launch_fa<T, 1, 4, false, false, true>(a, s);
+        return causal ? fa::launch_fa<T, NQS, NKS, true, true, true, SRES>(a, s)
+                      : fa::launch_fa<T, NQS, NKS, false, true, true, SRES>(a, s);
+    return causal ? fa::launch_fa<T, NQS, NKS, true, false, true>(a, s)
+                  : fa::launch_fa<T, NQS, NKS, false, false, true>(a, s);
 }
 
 // Head dims below the padded one and unaligned rows (guarded loads): two
@@ -321,21 +325,24 @@ hipError_t launch_fa_f32(const AttnArgs& a, bool causal, bool vec, hipStream_t s
     const bool small = n128 <= 64 && Sk > 128 && Sk <= 256;
     switch (fa_f32_padded_dim(a.D)) {
         case 32:
-            if (small) return launch_small<32>(a, causal, probs, s);
-            if (n128 <= 64 || (n128 <= 128 && Sk <= 256 && (causal || probs)))
-                return launch_shape<32, 1, 4, 1, 2>(a, causal, probs, s);
+            if (probs && Sk <= 256)
+                return n128 <= 128 && Sk > 128 ? launch_f32<32, 1, 4, 2>(a, causal, probs, s)
+                                               : launch_f32<32, 2, 2, 4>(a, causal, probs, s);
+            if (small) return launch_f32<32, 1, 4, 2>(a, causal, probs, s);
+            if (n128 <= 64 || (n128 <= 128 && Sk <= 256 && causal))
+                return launch_shape<32, 1, 4, 1>(a, causal, probs, s);
             if (n128 <= 128 && Sk > 256) return launch_shape<32, 2, 4, 1, 2>(a, causal, probs, s);
-            if (n128 <= 128 || (probs ? Sk <= 256 : causal && n128 <= 256))
-                return launch_shape<32, 2, 2, 2, 4>(a, causal, probs, s);
+            if (n128 <= 128 || (n128 <= 256 && causal && !probs)) return launch_shape<32, 2, 2, 2>(a, causal, probs, s);
             if (n128 >= 512 && Sk <= 256) return launch_shape<32, 4, 1, 2>(a, causal, probs, s);
-            return launch_shape<32, 4, 2, 1, 2>(a, causal, probs, s);
+            return launch_shape<32, 4, 2, 1>(a, causal, probs, s);
         case 64:
-            if (small) return launch_small<64>(a, causal, probs, s);
+            if (small) return launch_f32<64, 1, 4, 2>(a, causal, probs, s);
             if (n128 <= 128 && Sk > 256) return launch_shape<64, 2, 4, 1>(a, causal, probs, s);
             if (n128 <= 128 || (n128 <= 256 && (causal || (probs && Sk <= 256))))
                 return launch_shape<64, 2, 2, 1, 4>(a, causal, probs, s);
             if (n128 <= 256 || (causal && n128 <= 512 && Sk > 512))
                 return launch_shape<64, 4, 2, 1>(a, causal, probs, s);
+            if (Sk <= 256) return launch_shape<64, 4, 1, 2>(a, causal, probs, s);
             return launch_shape<64, 4, 1, 1>(a, causal, probs, s);
         case 128:
             if (n128 <= 128 || (n128 <= 256 && causal && Sk > 512)) return launch_shape<128, 2, 2, 1>(a, causal, probs, s);

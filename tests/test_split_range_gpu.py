@@ -28,7 +28,8 @@ pytestmark = pytest.mark.gpu
 # padded head dims and lengths that are no multiple of a tile
 SHAPES = [(1, 8, 256, 32), (2, 8, 300, 32), (16, 8, 200, 32), (64, 8, 130, 32), (1, 4, 256, 64), (2, 4, 333, 64),
           (20, 8, 257, 64), (70, 8, 100, 64), (2, 4, 200, 128), (20, 8, 190, 128), (70, 8, 129, 128), (2, 3, 70, 48),
-          (3, 3, 90, 96), (40, 8, 150, 80), (3, 2, 61, 20)]
+          (3, 3, 90, 96), (40, 8, 150, 80), (3, 2, 61, 20), (7, 8, 180, 32), (4, 8, 290, 32), (7, 8, 180, 64),
+          (6, 8, 600, 64), (12, 8, 170, 128)]
 
 
 def make(B, H, S, D, seed):
