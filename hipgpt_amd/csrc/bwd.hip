@@ -371,7 +371,7 @@ hipError_t launch_attn_bwd(const BwdArgs& a, hipStream_t s) {
             return n128 <= 128 || (a.causal && n128 <= 256) ? bwd::launch_terms<128, 2, 2, false>(a, s)
                                                             : bwd::launch_terms<128, 4, 2, false>(a, s);
         }
-        return bwd::launch_wide<256, 2, 4, 1>(a, s);
+        return bwd::launch_wide<256, 2, 4>(a, s);
     }
     if (a.D <= 32) return launch_dp<32>(a, s);
     if (a.D <= 64) return launch_dp<64>(a, s);

@@ -532,9 +532,9 @@ template <int DP, int NB, int DH, bool CAUSAL, bool RECOMP, bool TIGHT>
 struct TermPair {
     using Q = TermQ<DP, NB, DH, CAUSAL, RECOMP>;
     using KV = TermKV<DP, NB, DH, CAUSAL, RECOMP, RECOMP && TIGHT>;
-    using XQ = std::conditional_t<TIGHT, BwdQ<TIGHT ? DP : 32, NB, CAUSAL, RECOMP>, WideQ<DP, NB, DH, 1, CAUSAL, RECOMP>>;
+    using XQ = std::conditional_t<TIGHT, BwdQ<TIGHT ? DP : 32, NB, CAUSAL, RECOMP>, WideQ<DP, NB, DH, CAUSAL, RECOMP>>;
     using XKV =
-        std::conditional_t<TIGHT, BwdKV<TIGHT ? DP : 32, NB, CAUSAL, RECOMP>, WideKV<DP, NB, DH, 1, CAUSAL, RECOMP>>;
+        std::conditional_t<TIGHT, BwdKV<TIGHT ? DP : 32, NB, CAUSAL, RECOMP>, WideKV<DP, NB, DH, CAUSAL, RECOMP>>;
     static constexpr int QB = Q::LDS_BYTES > 4 * XQ::LDS_FLOATS ? Q::LDS_BYTES : 4 * XQ::LDS_FLOATS;
     static constexpr int KB = KV::LDS_BYTES > 4 * XKV::LDS_FLOATS ? KV::LDS_BYTES : 4 * XKV::LDS_FLOATS;
     static constexpr int NT = NB * DH * 64;

@@ -43,10 +43,9 @@ using fa::BK;
 using fa::halves_sum;
 
 // ----------------------------------------------------------------- dQ, Dq
-// Workgroup: NQB query sub-blocks x DH dim slices; NBUF stage buffers (2:
-// the next stage goes to the other buffer during the MFMAs; 1: it waits in
-// registers and is stored after a barrier).
-template <int DP, int NQB, int DH, int NBUF, bool CAUSAL, bool RECOMP>
+// Workgroup: NQB query sub-blocks x DH dim slices; one stage buffer, the next
+// stage waits in registers and is stored after a barrier.
+template <int DP, int NQB, int DH, bool CAUSAL, bool RECOMP>
 struct WideQ {
     using T = RowTiles<DP, DH>;
     static constexpr int NW = NQB * DH;
@@ -54,7 +53,7 @@ struct WideQ {
     static constexpr int STAGE = 2 * T::ROW;  // V, K (row-major)
     static constexpr int NACC = RECOMP ? 1 : 2;  // accumulators: A (, Bm)
     static constexpr int XCH = DH > 1 ? NW * 16 * 64 * (RECOMP ? 2 : 1) : 0;  // partial dP (, S') tiles
-    static constexpr int LDS_FLOATS = NBUF * STAGE + XCH;
+    static constexpr int LDS_FLOATS = STAGE + XCH;
 
     __device__ __forceinline__ static void run(const BwdArgs& a, float* lds, int nqb, int bh, int rank) {
         int tid = threadIdx.x;
@@ -103,7 +102,7 @@ struct WideQ {
         vl.init(a.v + base, a.ts, S, D);
         kl.init(a.k + base, a.ts, S, D);
         RowStage<DP, NT, 2> stg;
-        floatx4* const xch = reinterpret_cast<floatx4*>(lds + NBUF * STAGE);
+        floatx4* const xch = reinterpret_cast<floatx4*>(lds + STAGE);
 
         floatx16 acc[NACC][T::NDBW];  // A^T (recompute: dS K), Bm^T: [d][query]
 #pragma unroll
@@ -137,7 +136,7 @@ struct WideQ {
         }
         __syncthreads();
         for (int st = 0; st < nstages; ++st) {
-            const float* cur = lds + (NBUF == 2 ? (st & 1) * STAGE : 0);
+            const float* cur = lds;
             if (st + 1 < nstages) stg.load(vl, kl, (st + 1) * BK, D, tid);
             const bool act = st < wtiles;  // wave-uniform
             floatx16 dp;
@@ -190,15 +189,10 @@ struct WideQ {
                 ld += s;
                 T::template rchain<2>(acc, cur + T::ROW, x, c, hf, dh);  // A^T += K^T (P o dP)^T, Bm^T += K^T P^T
             }
-            if constexpr (NBUF == 2) {
-                if (st + 1 < nstages) stg.store(lds + ((st + 1) & 1) * STAGE, T::ROW, tid);
+            __syncthreads();
+            if (st + 1 < nstages) {
+                stg.store(lds, T::ROW, tid);
                 __syncthreads();
-            } else {
-                __syncthreads();
-                if (st + 1 < nstages) {
-                    stg.store(lds, T::ROW, tid);
-                    __syncthreads();
-                }
             }
         }
 
@@ -225,7 +219,7 @@ struct WideQ {
 };
 
 // ----------------------------------------------------------------- dK, dV
-template <int DP, int NKB, int DH, int NBUF, bool CAUSAL, bool RECOMP>
+template <int DP, int NKB, int DH, bool CAUSAL, bool RECOMP>
 struct WideKV {
     using T = RowTiles<DP, DH>;
     static constexpr int NW = NKB * DH;
@@ -234,7 +228,7 @@ struct WideKV {
     static constexpr int LSE_OFF = DQ_OFF + BK;
     static constexpr int STAGE = 2 * T::ROW + BK + (RECOMP ? BK : 0);  // dO, Q (row-major), Dq (, lse')
     static constexpr int XCH = DH > 1 ? NW * 16 * 64 * (RECOMP ? 2 : 1) : 0;  // partial dP (, S') tiles
-    static constexpr int LDS_FLOATS = NBUF * STAGE + XCH;
+    static constexpr int LDS_FLOATS = STAGE + XCH;
     static_assert(STAGE % 4 == 0, "16-byte aligned stage buffers");
 
     __device__ __forceinline__ static void run(const BwdArgs& a, float* lds, int bh, int rank) {
@@ -271,7 +265,7 @@ struct WideKV {
         RowStage<DP, NT, 2> stg;
         float dqs = 0.f;
         float lses = 0.f;  // recompute mode: lse' of the staged row (+inf past the last row: P = 0)
-        floatx4* const xch = reinterpret_cast<floatx4*>(lds + NBUF * STAGE);
+        floatx4* const xch = reinterpret_cast<floatx4*>(lds + STAGE);
 
         floatx16 acc[2][T::NDBW];  // dV^T, dK^T (unscaled): [d][key]
 #pragma unroll
@@ -313,7 +307,7 @@ struct WideKV {
         }
         __syncthreads();
         for (int st = 0; st < nstages; ++st) {
-            const float* cur = lds + (NBUF == 2 ? (st & 1) * STAGE : 0);
+            const float* cur = lds;
             if (st + 1 < nstages) load(st + 1);
             const int it = it0 + st;
             const bool act = it >= wit0;  // wave-uniform
@@ -367,15 +361,10 @@ struct WideKV {
                 T::template rchain<1>(&acc[0], cur, &x[0], c, hf, dh);           // dV^T += dO^T P
                 T::template rchain<1>(&acc[1], cur + T::ROW, &x[1], c, hf, dh);  // dK^T += Q^T dS
             }
-            if constexpr (NBUF == 2) {
-                if (st + 1 < nstages) store(lds + ((st + 1) & 1) * STAGE);
+            __syncthreads();
+            if (st + 1 < nstages) {
+                store(lds);
                 __syncthreads();
-            } else {
-                __syncthreads();
-                if (st + 1 < nstages) {
-                    store(lds);
-                    __syncthreads();
-                }
             }
         }
 
@@ -399,17 +388,17 @@ struct WideKV {
     }
 };
 
-template <int DP, int NQB, int DH, int NBUF, bool CAUSAL, bool RECOMP>
+template <int DP, int NQB, int DH, bool CAUSAL, bool RECOMP>
 __global__ __launch_bounds__(NQB* DH * 64) void bwd_wide_q_kernel(BwdArgs a, int nqb) {
-    using K = WideQ<DP, NQB, DH, NBUF, CAUSAL, RECOMP>;
+    using K = WideQ<DP, NQB, DH, CAUSAL, RECOMP>;
     __shared__ __attribute__((aligned(16))) float lds[K::LDS_FLOATS];
     const int BH = a.B * a.H;
     K::run(a, lds, nqb, blockIdx.x % BH, blockIdx.x / BH);
 }
 
-template <int DP, int NKB, int DH, int NBUF, bool CAUSAL, bool RECOMP>
+template <int DP, int NKB, int DH, bool CAUSAL, bool RECOMP>
 __global__ __launch_bounds__(NKB* DH * 64) void bwd_wide_kv_kernel(BwdArgs a) {
-    using K = WideKV<DP, NKB, DH, NBUF, CAUSAL, RECOMP>;
+    using K = WideKV<DP, NKB, DH, CAUSAL, RECOMP>;
     __shared__ __attribute__((aligned(16))) float lds[K::LDS_FLOATS];
     const int BH = a.B * a.H;
     K::run(a, lds, blockIdx.x % BH, blockIdx.x / BH);
@@ -418,30 +407,30 @@ __global__ __launch_bounds__(NKB* DH * 64) void bwd_wide_kv_kernel(BwdArgs a) {
 // Both kernels of one problem (the second reads the first's Dq).  Blocks
 // b run (b, h) = b mod B*H at launch rank b / B*H: the heaviest causal blocks
 // of every (b, h) first.
-template <int DP, int NB, int DH, int NBUF, bool CAUSAL, bool RECOMP>
+template <int DP, int NB, int DH, bool CAUSAL, bool RECOMP>
 hipError_t launch_wide_mode(const BwdArgs& a, hipStream_t s) {
     const int BH = a.B * a.H;
     const int nb = (a.S + NB * BK - 1) / (NB * BK);
     const int64_t g = (int64_t)nb * BH;
     if (g <= 0 || g > 0x7fffffff) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL((bwd_wide_q_kernel<DP, NB, DH, NBUF, CAUSAL, RECOMP>), dim3((unsigned)g), dim3(NB * DH * 64), 0,
+    hipLaunchKernelGGL((bwd_wide_q_kernel<DP, NB, DH, CAUSAL, RECOMP>), dim3((unsigned)g), dim3(NB * DH * 64), 0,
                        s, a, nb);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((bwd_wide_kv_kernel<DP, NB, DH, NBUF, CAUSAL, RECOMP>), dim3((unsigned)g), dim3(NB * DH * 64),
+    hipLaunchKernelGGL((bwd_wide_kv_kernel<DP, NB, DH, CAUSAL, RECOMP>), dim3((unsigned)g), dim3(NB * DH * 64),
                        0, s, a);
     return hipGetLastError();
 }
 
 // Stored probs, or (probs == nullptr) recompute mode from a.o and a.lse; both
 // need the B*H*S workspace a.dvec.
-template <int DP, int NB, int DH, int NBUF>
+template <int DP, int NB, int DH>
 hipError_t launch_wide(const BwdArgs& a, hipStream_t s) {
     if (!a.probs)
-        return a.causal ? launch_wide_mode<DP, NB, DH, NBUF, true, true>(a, s)
-                        : launch_wide_mode<DP, NB, DH, NBUF, false, true>(a, s);
-    return a.causal ? launch_wide_mode<DP, NB, DH, NBUF, true, false>(a, s)
-                    : launch_wide_mode<DP, NB, DH, NBUF, false, false>(a, s);
+        return a.causal ? launch_wide_mode<DP, NB, DH, true, true>(a, s)
+                        : launch_wide_mode<DP, NB, DH, false, true>(a, s);
+    return a.causal ? launch_wide_mode<DP, NB, DH, true, false>(a, s)
+                    : launch_wide_mode<DP, NB, DH, false, false>(a, s);
 }
 
 }  // namespace bwd

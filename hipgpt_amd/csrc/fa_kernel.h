@@ -8,8 +8,8 @@
 //     key tile starting at tile ks, so a long causal row is split over NKS
 //     waves (balance) and the CU holds NKS times more waves (latency hiding).
 //   * One stage = NKS key tiles of 32 rows, staged global -> registers ->
-//     LDS (K row-major, V transposed), double buffered, one barrier per
-//     stage; the next stage's global loads are in flight during compute.
+//     LDS, in two buffers (one barrier per stage) or one (two barriers); the
+//     next stage's global loads are in flight during compute.
 //   * Per tile: S^T = K Q^T (32x32 MFMA accumulator, layout in fa_common.h),
 //     mask, online softmax in the log2 domain, O^T += V^T P^T with P taken
 //     straight from the accumulator registers.
@@ -513,9 +513,8 @@ struct FaKernel {
         };
 
         // Stage pipeline: stage i+1 is loaded into registers while stage i is
-        // computed, then written to the other LDS buffer.  (Two stages of
-        // register prefetch measured no faster at any head dim and cost an
-        // occupancy step at D = 32.)
+        // computed, then written to the other LDS buffer or, with one, to the same
+        // after a barrier.
         // With probs, the max/sum sweep (MODE 1) requests the probs sweep's first stage during its last one, so
         // the probs sweep (MODE 2) starts from registers instead of a memory round trip.
         constexpr bool WV2 = true, WK2 = !SPILL;  // what the probs sweep stages
