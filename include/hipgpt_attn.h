@@ -121,7 +121,7 @@ int hipgpt_attn_qkv_planar(const float* d_qkv, float* d_output,
  * three bf16 terms, six bf16 MFMAs make a product (off by at most 2^-24 of
  * itself) and sums are fp32; results that are not finite that way (infinities,
  * NaN, operands of 2^103, sums of 2^80 and more) are formed again on fp32 MFMA.
- * The backward (D <= 128) and the projections do the same.  o may be q.
+ * The backward (D <= 128) and the projections do the same.  At D <= 128 o may be q.
  * bf16 inputs are computed with bf16 MFMA and fp32 accumulation, D in
  * {32, 64, 128}, 16-byte aligned rows (strides multiple of 8). */
 int hipgpt_attn_fwd(const void* q, const void* k, const void* v, float* o,
